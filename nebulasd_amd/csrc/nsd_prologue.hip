@@ -85,7 +85,8 @@ __global__ __launch_bounds__(256) void store_kv_prefill_kernel(
   }
 }
 
-// One wave per row of `hidden` values.  Mirrors _fwd_rmsnorm (rmsnorm.py:5-24).
+// RMSNorm, mirroring _fwd_rmsnorm (rmsnorm.py:5-24).  One wave per row of any
+// width and alignment; the vector kernels below take what they can.
 __global__ __launch_bounds__(256) void rmsnorm_kernel(f16* __restrict__ x, const f16* __restrict__ w,
                                                       int64_t n_rows, int64_t hidden, float eps) {
   const int lane = threadIdx.x & 63;
@@ -102,8 +103,91 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(f16* __restrict__ x, const
   for (int64_t i = lane; i < hidden; i += kWave) xr[i] = (f16)((float)xr[i] * rstd * (float)w[i]);
 }
 
+// Sum over the 16 lanes of a DPP row, in every lane: neighbours, pairs, then
+// the two mirrors (each lane's partner there holds another quad's, another
+// half's sum).
+template <int CTRL>
+__device__ inline float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ inline float row16_sum(float v) {
+  v = dpp_add<0xB1>(v);    // quad_perm [1,0,3,2]
+  v = dpp_add<0x4E>(v);    // quad_perm [2,3,0,1]
+  v = dpp_add<0x141>(v);   // row_half_mirror
+  return dpp_add<0x140>(v);  // row_mirror
+}
+
+__device__ inline f16x8 h8(u32x4 v) { return __builtin_bit_cast(f16x8, v); }
+__device__ inline u32x4 u4(f16x8 v) { return __builtin_bit_cast(u32x4, v); }
+__device__ inline float sum_squares(f16x8 v) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss += (float)v[e] * (float)v[e];
+  return ss;
+}
+__device__ inline f16x8 scaled(f16x8 v, float rstd, f16x8 w) {
+  f16x8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = (f16)((float)v[e] * rstd * (float)w[e]);
+  return o;
+}
+
+// Head rows (the QK-norm): bound by memory, one read and one write.  16 lanes
+// of 16 bytes hold a row, so a wave covers four and no lane idles, and each
+// thread takes kHeadRows rows with their loads in flight together.  Before,
+// a wave read one row in 2-byte lanes: 150k rows 43.8 us, now 14.6 (5.3 TB/s).
+constexpr int kHeadRows = 4;
+__global__ __launch_bounds__(256) void rmsnorm_heads_kernel(u32x4* __restrict__ x, const u32x4* __restrict__ w,
+                                                            int64_t n_rows, float eps) {
+  const int c = threadIdx.x & 15;
+  const int64_t row0 = (int64_t)blockIdx.x * (16 * kHeadRows) + (threadIdx.x >> 4);
+  const f16x8 wv = h8(w[c]);
+  u32x4 v[kHeadRows];
+#pragma unroll
+  for (int u = 0; u < kHeadRows; ++u) {
+    const int64_t row = row0 + 16 * u;
+    v[u] = x[(row < n_rows ? row : n_rows - 1) * kUnits + c];
+  }
+#pragma unroll
+  for (int u = 0; u < kHeadRows; ++u) {
+    const int64_t row = row0 + 16 * u;
+    const f16x8 xv = h8(v[u]);
+    const float rstd = 1.f / sqrtf(row16_sum(sum_squares(xv)) / (float)D + eps);
+    if (row < n_rows) x[row * kUnits + c] = u4(scaled(xv, rstd, wv));
+  }
+}
+
+// Rows of a model's hidden size (the final norm): one workgroup per row, the
+// row in registers between the sum and the scaled store.
+constexpr int kRowVecs = 4;  // 16-byte vectors per thread: hidden <= 8192
+__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(u32x4* __restrict__ x, const u32x4* __restrict__ w,
+                                                           int nvec, float eps) {
+  __shared__ float s_part[4];
+  u32x4* xr = x + (int64_t)blockIdx.x * nvec;
+  u32x4 v[kRowVecs];
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < kRowVecs; ++j) {
+    const int i = threadIdx.x + 256 * j;
+    if (i < nvec) {
+      v[j] = xr[i];
+      ss += sum_squares(h8(v[j]));
+    }
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float rstd = 1.f / sqrtf(((s_part[0] + s_part[1]) + (s_part[2] + s_part[3])) / (float)(8 * nvec) + eps);
+#pragma unroll
+  for (int j = 0; j < kRowVecs; ++j) {
+    const int i = threadIdx.x + 256 * j;
+    if (i < nvec) xr[i] = u4(scaled(h8(v[j]), rstd, h8(w[i])));
+  }
+}
+
 // One wave per (token, head); heads [0, Hq) rotate q, [Hq, Hq+Hkv) rotate k.
 // Mirrors _fwd_rotary_embedding (rotary_emb.py:7-42) with fp32 arithmetic.
+// Any head_dim and alignment; rope_heads_kernel takes heads of 128.
 __global__ __launch_bounds__(256) void rope_kernel(f16* __restrict__ q, f16* __restrict__ k,
                                                    const f16* __restrict__ cos_t,
                                                    const f16* __restrict__ sin_t, int64_t n_tokens,
@@ -121,6 +205,46 @@ __global__ __launch_bounds__(256) void rope_kernel(f16* __restrict__ q, f16* __r
     const float x0 = (float)x[j], x1 = (float)x[j + half];
     x[j] = (f16)(x0 * c - x1 * s);
     x[j + half] = (f16)(x0 * s + x1 * c);
+  }
+}
+
+// The same for heads of 128, bit for bit: bound by memory, so eight lanes
+// hold a head's two halves in 16-byte vectors (8 heads a wave) and a thread
+// keeps kRopeHeads heads' loads in flight.  Before, 2-byte lanes: 9374 tokens
+// x 24 heads 38.8 us, now 23.2 (4.9 TB/s).
+constexpr int kRopeHeads = 4;
+__global__ __launch_bounds__(256) void rope_heads_kernel(u32x4* __restrict__ q, u32x4* __restrict__ k,
+                                                         const u32x4* __restrict__ cos_t,
+                                                         const u32x4* __restrict__ sin_t, uint32_t n_heads,
+                                                         uint32_t hq, uint32_t hkv) {
+  constexpr int H = kUnits / 2;  // vectors of half a head
+  const uint32_t c = threadIdx.x & (H - 1);
+  const uint32_t i0 = blockIdx.x * (32u * kRopeHeads) + (threadIdx.x >> 3);
+  u32x4* at[kRopeHeads];
+  u32x4 lo[kRopeHeads], hi[kRopeHeads], cv[kRopeHeads], sv[kRopeHeads];
+#pragma unroll
+  for (int u = 0; u < kRopeHeads; ++u) {
+    const uint32_t i = min(i0 + 32 * u, n_heads - 1);  // past the end: the last head, not stored
+    const uint32_t t = i / (hq + hkv), hd = i - t * (hq + hkv);
+    at[u] = (hd < hq ? q + ((int64_t)t * hq + hd) * kUnits : k + ((int64_t)t * hkv + (hd - hq)) * kUnits) + c;
+    lo[u] = at[u][0];
+    hi[u] = at[u][H];
+    cv[u] = cos_t[(int64_t)t * H + c];
+    sv[u] = sin_t[(int64_t)t * H + c];
+  }
+#pragma unroll
+  for (int u = 0; u < kRopeHeads; ++u) {
+    if (i0 + 32 * u >= n_heads) break;
+    const f16x8 a = h8(lo[u]), b = h8(hi[u]), cs = h8(cv[u]), sn = h8(sv[u]);
+    f16x8 o0, o1;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x0 = (float)a[e], x1 = (float)b[e], cc = (float)cs[e], ss = (float)sn[e];
+      o0[e] = (f16)(x0 * cc - x1 * ss);
+      o1[e] = (f16)(x0 * ss + x1 * cc);
+    }
+    at[u][0] = u4(o0);
+    at[u][H] = u4(o1);
   }
 }
 
@@ -250,6 +374,19 @@ extern "C" int nsd_rmsnorm_inplace(void* x, const void* w, int64_t n_rows, int64
                                              (long long)n_rows, (long long)hidden);
   if (n_rows == 0) return NSD_OK;
   if (x == nullptr || w == nullptr) return fail(NSD_ERR_INVALID, "rmsnorm: null pointer");
+  const bool vectors = aligned16(x) && aligned16(w) && n_rows <= INT32_MAX;
+  if (vectors && hidden == D) {
+    hipLaunchKernelGGL(rmsnorm_heads_kernel, dim3((unsigned)((n_rows + 16 * kHeadRows - 1) / (16 * kHeadRows))),
+                       dim3(256), 0, as_stream(stream), static_cast<u32x4*>(x), static_cast<const u32x4*>(w), n_rows,
+                       eps);
+    return launch_status("rmsnorm");
+  }
+  // a workgroup per row from the width on where its 256 threads have a vector each
+  if (vectors && hidden % 8 == 0 && hidden >= 1024 && hidden <= 8 * 256 * kRowVecs) {
+    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)n_rows), dim3(256), 0, as_stream(stream),
+                       static_cast<u32x4*>(x), static_cast<const u32x4*>(w), (int)(hidden / 8), eps);
+    return launch_status("rmsnorm");
+  }
   const unsigned grid = (unsigned)((n_rows + 3) / 4);
   hipLaunchKernelGGL(rmsnorm_kernel, dim3(grid), dim3(256), 0, as_stream(stream),
                      static_cast<f16*>(x), static_cast<const f16*>(w), n_rows, hidden, eps);
@@ -265,6 +402,14 @@ extern "C" int nsd_rotary_embedding_inplace(void* q, void* k, const void* cos_ta
   if (n_tokens == 0) return NSD_OK;
   if (!q || !k || !cos_table || !sin_table) return fail(NSD_ERR_INVALID, "rope: null pointer");
   const int64_t waves = n_tokens * (num_q_heads + num_kv_heads);
+  if (head_dim == D && waves <= INT32_MAX && aligned16(q) && aligned16(k) && aligned16(cos_table) &&
+      aligned16(sin_table)) {
+    hipLaunchKernelGGL(rope_heads_kernel, dim3((unsigned)((waves + 32 * kRopeHeads - 1) / (32 * kRopeHeads))),
+                       dim3(256), 0, as_stream(stream), static_cast<u32x4*>(q), static_cast<u32x4*>(k),
+                       static_cast<const u32x4*>(cos_table), static_cast<const u32x4*>(sin_table), (uint32_t)waves,
+                       (uint32_t)num_q_heads, (uint32_t)num_kv_heads);
+    return launch_status("rope");
+  }
   hipLaunchKernelGGL(rope_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
                      as_stream(stream), static_cast<f16*>(q), static_cast<f16*>(k),
                      static_cast<const f16*>(cos_table), static_cast<const f16*>(sin_table),

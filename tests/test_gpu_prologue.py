@@ -124,6 +124,53 @@ def test_rope_matches_oracle(gpu):
     ulp_close(k.cpu().numpy(), wk, "rope k")
 
 
+def placed(t: torch.Tensor, offset: int):
+    """A copy of t `offset` elements past a 16-byte boundary, and the buffer around it (guards of 7)."""
+    buf = torch.full((t.numel() + offset + 7,), 7.0, dtype=t.dtype, device=t.device)
+    view = buf[offset:offset + t.numel()].view(t.shape)
+    view.copy_(t)
+    return view, buf
+
+
+def guards_kept(buf, n, offset):
+    return bool((buf[:offset] == 7).all() and (buf[offset + n:] == 7).all())
+
+
+@pytest.mark.parametrize("rows,hidden,offset", [
+    (1, 128, 0), (63, 128, 0), (64, 128, 0), (65, 128, 0), (65, 128, 1),      # head rows: around a workgroup's 64
+    (3, 1016, 0), (3, 1024, 0), (5, 4096, 0), (2, 8192, 0), (2, 8200, 0), (3, 4096, 1), (2, 100, 0)])
+def test_rmsnorm_widths_and_alignments(gpu, rows, hidden, offset):
+    g = torch.Generator(device=gpu).manual_seed(rows + hidden)
+    x, buf = placed((torch.randn((rows, hidden), device=gpu, generator=g) * 3).half(), offset)
+    w = (torch.rand(hidden, device=gpu, generator=g) + 0.5).half()
+    want = oracle.rmsnorm(x.cpu().numpy(), w.cpu().numpy(), 1e-6)
+    rmsnorm_inplace(x, w, 1e-6)
+    ulp_close(x.cpu().numpy(), want, "rmsnorm")
+    assert guards_kept(buf, x.numel(), offset)
+
+
+@pytest.mark.parametrize("tokens,hq,hkv,d,offset", [
+    (1, 1, 1, 128, 0), (43, 2, 1, 128, 0), (32, 3, 1, 128, 0), (127, 1, 1, 128, 0), (300, 32, 8, 128, 0),
+    (43, 2, 1, 128, 1), (9, 4, 2, 64, 0)])
+def test_rope_head_counts_and_alignments(gpu, tokens, hq, hkv, d, offset):
+    g = torch.Generator(device=gpu).manual_seed(tokens + hq)
+    cos_c, sin_c = rope_cache(d, 1e6, 4096, gpu)
+    pos = torch.randint(0, 4096, (tokens,), device=gpu, generator=g)
+    q, qbuf = placed(torch.randn((tokens, hq, d), device=gpu, generator=g).half(), offset)
+    k, kbuf = placed(torch.randn((tokens, hkv, d), device=gpu, generator=g).half(), offset)
+
+    class S:
+        position_cos = cos_c[pos].contiguous()
+        position_sin = sin_c[pos].contiguous()
+
+    wq = oracle.rope(q.cpu().numpy(), S.position_cos.cpu().numpy(), S.position_sin.cpu().numpy())
+    wk = oracle.rope(k.cpu().numpy(), S.position_cos.cpu().numpy(), S.position_sin.cpu().numpy())
+    rotary_embedding_inplace(q, k, S)
+    ulp_close(q.cpu().numpy(), wq, "rope q")
+    ulp_close(k.cpu().numpy(), wk, "rope k")
+    assert guards_kept(qbuf, q.numel(), offset) and guards_kept(kbuf, k.numel(), offset)
+
+
 def test_rope_table_matches_oracle(gpu):
     """The table is built in fp32 (model.py:242-252): the argument t*inv_freq
     carries up to ~2 fp32 roundings of |t| (and pow may differ by an ulp
