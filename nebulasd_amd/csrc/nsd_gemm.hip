@@ -1,9 +1,10 @@
 // Projection GEMMs of decode/verify batches for gfx950 (MI355X).
 //
 // y[rows, n] = x[rows, k] . W[n, k]^T (fp16 in, fp32 sums) for the q/k/v, O
-// and down projections of a layer at decode/verify batch sizes (rows <= 128).
-// The weight is the whole of the traffic (x is at most 3 MB and stays in L2),
-// so the kernel is a stream of W through the compute units:
+// and down projections of a layer at decode/verify batch sizes (rows <= 128),
+// and the FFN's up/gate projection with its SiLU-and-mul.  The weight is the
+// whole of the traffic (x is at most 3 MB and stays in L2), so the kernels are
+// a stream of W through the compute units:
 //
 //   - the work is cut into (n-tile of TN columns, k-range) units, one
 //     workgroup each, about one per compute unit: TN columns over all of k
@@ -13,26 +14,27 @@
 //     add-RMSNorm, the QK-norm/RoPE/KV-store prologue, or a small sum pass)
 //     adds the splits in split order and rounds to fp16 once, which is the
 //     GEMM output rounding of F.linear;
-//   - a workgroup streams its unit in steps of 128 k through a ring of LDS
-//     slots filled by global_load_lds_dwordx4 (each instruction brings four
-//     256-byte row chunks), a slot holding the step's TN weight rows and the
-//     step's x rows, with two steps in flight; rows are XOR-swizzled per
-//     16-byte chunk so the 16 rows an MFMA operand read touches hit distinct
-//     banks;
-//   - v_mfma_f32_16x16x32_f16 with A = weight rows, B = x rows: for TN >= 64
-//     each wave owns TN/64 of the 16-column n-tiles over the whole step, for
-//     TN = 16 and 32 each wave owns one of the step's four 32-k sub-steps
-//     over every output tile and the four waves' sums are added in LDS, in
-//     wave order, at the end;
-//   - a gated unit serves the FFN's up/gate projection: 48 up and the
-//     matching 48 gate rows over all of k, the SiLU-and-mul applied to the
-//     accumulators, fp16 output (no partials).
+//   - a gated unit (the up/gate projection) streams 16 p up rows and the
+//     matching gate rows over all of k, applies the SiLU-and-mul to its
+//     accumulators and writes fp16 (no partials);
+//   - W and x arrive in LDS slots by global_load_lds_dwordx4; rows are
+//     XOR-swizzled per 16-byte chunk so the 16 rows an MFMA operand read
+//     touches hit distinct banks; v_mfma_f32_16x16x32_f16 with A = weight
+//     rows, B = x rows;
+//   - stream_gemm_kernel (gated units, and columns tiles of 64 and more):
+//     four waves only load, the others only compute, so the stream runs on
+//     under the arithmetic; linear_partials_kernel (column tiles of 16 and
+//     32, the small models' shapes, where a unit is a few steps long and the
+//     launch is most of the time): every wave does both.
 //
-// Measured on MI355X against hipBLASLt (the library F.linear uses), µs per
-// call with the weights rotated past the MALL: Qwen3-8B at 80 rows, O
-// 4096x4096 10.5 (16.6), down 12288 -> 4096 23.6-25 (40.9), q/k/v 4096 ->
-// 6144 15.5 (23.2); Qwen3-0.6B at 64 rows, q/k/v 5.4 (11.6), O 4.2 (10.6),
-// down 4.9 (9.3).
+// Measured on MI355X, us per call with the weights rotated past the MALL,
+// before (every wave loading and computing) -> now: Qwen3-8B up/gate 24576 x
+// 4096 at 16 / 80 / 128 rows 37.7 / 42.3 / 57.6 -> 34.6 / 36.6 / 42.8 (the W
+// stream alone 33.5); q/k/v 4096 -> 6144 10.4 / 14.4 / 18.1 -> 10.3 / 13.6 /
+// 16.2; down 12288 -> 4096 17.1 / 22.5 / 34.9 -> 17.2 / 21.5 / 26.1; O 4096 ->
+// 4096 7.3 / 9.9 / 13.5 -> 7.2 / 9.4 / 11.1.  Qwen3-0.6B at 64 rows: up/gate
+// 9.8 -> 6.0; q/k/v 4.9, O 4.0, down 4.8 stay with the small-tile kernel,
+// which the split roles did not beat there.
 #include <algorithm>
 #include <atomic>
 
@@ -44,7 +46,7 @@ namespace {
 constexpr int kKStep = 128;                 // k per ring step
 constexpr int kStepRowBytes = kKStep * 2;   // one row's chunk of a step
 constexpr int kGemmThreads = 256;
-constexpr int kGemmLds = 156 * 1024;        // LDS one workgroup may use
+constexpr int kGemmLds = 160 * 1024;        // LDS one workgroup may use
 constexpr int kMaxSplits = 8;
 constexpr int kMaxRowTiles = 8;             // 128 rows
 
@@ -74,53 +76,40 @@ __device__ inline void gemm_wait() {
 }
 __device__ inline void gemm_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-// GATED: the FFN's up/gate projection with SiLU-and-mul in the epilogue:
-// the unit's TN weight rows are TN/2 up rows then the same TN/2 gate rows
-// (W = [up; gate], 2 * n rows), over all of k, and the unit writes fp16
-// h = fp16(up) * fp16(silu(fp16(gate))) for its TN/2 columns.
+// ---- small column tiles ----------------------------------------------------
 //
-// How the four waves share a step's MFMAs (kMode): 0 -- each wave one of the
-// four 32-k sub-steps over every output tile, summed across waves in LDS at
-// the end (TN 16, 32); 1 -- each wave TN/64 of the 16-column tiles over the
-// whole step (TN >= 64); 2 -- GATED: wave w (< TN/32) the up tile w and its
-// gate tile over the whole step, so the SiLU-and-mul needs no exchange.
-template <int MT, int TN, bool GATED = false>
+// Each of the four waves brings its share of a step (128 k: TN weight rows
+// and the x rows) and computes one of its four 32-k sub-steps over every
+// output tile; the waves' sums are added in LDS, in wave order, at the end.
+template <int MT, int TN>
 struct LinearShape {
   static constexpr int kRows = TN + 16 * MT;            // rows of one slot: weight, then x
   static constexpr int kSlot = kRows * kStepRowBytes;
-  static constexpr int kRing = 3 * kSlot <= kGemmLds ? 3 : 2;
+  static constexpr int kRing = 3;                       // two steps in flight
   static constexpr int kLds = kRing * kSlot;
   static constexpr int kDmaPerWave = kRows / 16;        // 4 rows per instruction, 4 waves
-  static constexpr int kMode = GATED ? 2 : TN >= 64 ? 1 : 0;
-  static_assert(kRing * kSlot <= kGemmLds, "ring");
-  static_assert(kMode != 0 || 4 * (TN / 16) * MT * 1024 <= kLds, "reduction buffer");
-  static_assert(kMode != 2 || (TN / 32 <= 4 && TN % 32 == 0), "one up/gate tile pair per wave");
+  static_assert(kLds <= kGemmLds, "ring");
+  static_assert(4 * (TN / 16) * MT * 1024 <= kLds, "reduction buffer");
 };
 
 // Unit u = (n-tile u % n_tiles, split u / n_tiles); split s covers steps
 // [s T / splits, (s+1) T / splits) of the T = k / 128 steps.
-template <int MT, int TN, bool GATED = false>
+template <int MT, int TN>
 __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16* __restrict__ x,
                                                                        const f16* __restrict__ w,
                                                                        float* __restrict__ part, int rows,
-                                                                       int n, int k, int splits,
-                                                                       int n_tiles, f16* __restrict__ y) {
-  using S = LinearShape<MT, TN, GATED>;
+                                                                       int n, int k, int splits, int n_tiles) {
+  using S = LinearShape<MT, TN>;
   constexpr int R = S::kRing;
   constexpr int NI = S::kDmaPerWave;
   constexpr int NJ = TN / 16;
-  constexpr int M = S::kMode;
-  constexpr int NJW = M == 1 ? NJ / 4 : M == 2 ? 2 : NJ;  // n-tiles per wave
-  constexpr int KSUB = M == 0 ? 1 : 4;                     // 32-k sub-steps per wave per step
   extern __shared__ __align__(16) char smem_raw[];
   lds_char* ring = (lds_char*)smem_raw;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lg = lane >> 4;
   const int nt = blockIdx.x % n_tiles, split = blockIdx.x / n_tiles;
-  const int n0 = nt * (GATED ? TN / 2 : TN);
-  const bool computes = M != 2 || wave < NJ / 2;
-  auto tile_of = [&](int j) { return M == 1 ? wave * NJW + j : M == 2 ? wave + j * (NJ / 2) : j; };
+  const int n0 = nt * TN;
   const int T = k / kKStep;
   const int t0 = (int)((int64_t)split * T / splits);
   const int steps = (int)((int64_t)(split + 1) * T / splits) - t0;
@@ -132,9 +121,7 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
   for (int i = 0; i < NI; ++i) {
     const int row = (4 * i + wave) * 4 + (lane >> 4);
     const int chunk = (lane & 15) ^ chunk_swizzle(row);
-    // weight row of slot row `row` (GATED: up rows, then the gate rows n further on)
-    const int wrow = !GATED || row < TN / 2 ? n0 + row : n + n0 + row - TN / 2;
-    const f16* base = row < TN ? w + (int64_t)wrow * k
+    const f16* base = row < TN ? w + (int64_t)(n0 + row) * k
                                : x + (int64_t)(row - TN < rows ? row - TN : rows - 1) * k;  // pad rows: a real row
     src[i] = base + (int64_t)t0 * kKStep + chunk * 8;
   }
@@ -145,9 +132,9 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
       gemm_dma<(i < TN / 16)>((uint32_t)(uintptr_t)(slot + (4 * i + wave) * 1024), src[i] + (int64_t)t * kKStep);
     });
   };
-  f32x4 acc[NJW][MT];
+  f32x4 acc[NJ][MT];
 #pragma unroll
-  for (int j = 0; j < NJW; ++j)
+  for (int j = 0; j < NJ; ++j)
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -161,70 +148,254 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
     gemm_barrier();
     if (issued < steps) issue(issued++);
     const lds_char* sl = ring + (t % R) * S::kSlot;
-    if (!computes) continue;
+    const int ch = 4 * wave + lg;  // lane group's 8 k of the sub-step
+    f16x8 a[NJ], b[MT];
 #pragma unroll
-    for (int kk = 0; kk < KSUB; ++kk) {
-      const int ch = 4 * (M == 0 ? wave : kk) + lg;  // lane group's 8 k of the sub-step
-      f16x8 a[NJW], b[MT];
-#pragma unroll
-      for (int j = 0; j < NJW; ++j) {
-        const int row = 16 * tile_of(j) + lr;
-        a[j] = *(const lds_f16x8*)(sl + row * kStepRowBytes + ((ch ^ chunk_swizzle(row)) << 4));
-      }
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int row = TN + 16 * i + lr;
-        b[i] = *(const lds_f16x8*)(sl + row * kStepRowBytes + ((ch ^ chunk_swizzle(row)) << 4));
-      }
-#pragma unroll
-      for (int j = 0; j < NJW; ++j)
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[j][i] = mfma_k32(a[j], b[i], acc[j][i]);
+    for (int j = 0; j < NJ; ++j) {
+      const int row = 16 * j + lr;
+      a[j] = *(const lds_f16x8*)(sl + row * kStepRowBytes + ((ch ^ chunk_swizzle(row)) << 4));
     }
-  }
-  // lane (lg, lr) holds columns 4lg .. 4lg+3 of an n-tile for row lr of an
-  // m-tile: 16 contiguous bytes of the partial row (no partials when gated)
-  float* out = GATED ? nullptr : part + (int64_t)split * rows * n;
-  auto store = [&](int j, int i, f32x4 v) {
-    const int m = 16 * i + lr;
-    if (m < rows) *reinterpret_cast<f32x4*>(out + (int64_t)m * n + n0 + 16 * j + 4 * lg) = v;
-  };
-  if constexpr (M == 1) {
-#pragma unroll
-    for (int j = 0; j < NJW; ++j)
-#pragma unroll
-      for (int i = 0; i < MT; ++i) store(tile_of(j), i, acc[j][i]);
-  } else if constexpr (M == 2) {
-    // up tile `wave` and its gate tile leave the same lane layout: the
-    // SiLU-and-mul of silu_and_mul_kernel on the fp16-rounded sums
-    if (!computes) return;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
-      const int m = 16 * i + lr;
-      if (m >= rows) continue;
-      f16x4 h;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const f16 up = (f16)acc[0][i][e];
-        const float gf = (float)(f16)acc[1][i][e];
-        const f16 sg = (f16)(gf / (1.f + expf(-gf)));
-        h[e] = (f16)((float)up * (float)sg);
-      }
-      *reinterpret_cast<f16x4*>(y + (int64_t)m * n + n0 + 16 * wave + 4 * lg) = h;
+      const int row = TN + 16 * i + lr;
+      b[i] = *(const lds_f16x8*)(sl + row * kStepRowBytes + ((ch ^ chunk_swizzle(row)) << 4));
     }
-  } else {
-    __syncthreads();  // the ring is drained: its LDS holds the waves' sums
-    f32x4* red = reinterpret_cast<f32x4*>(smem_raw);  // [wave][tile][lane]
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
-      for (int i = 0; i < MT; ++i) red[(wave * NJ * MT + j * MT + i) * 64 + lane] = acc[j][i];
-    __syncthreads();
-    for (int tile = wave; tile < NJ * MT; tile += 4) {
-      f32x4 v = red[tile * 64 + lane];
+      for (int i = 0; i < MT; ++i) acc[j][i] = mfma_k32(a[j], b[i], acc[j][i]);
+  }
+  // lane (lg, lr) holds columns 4lg .. 4lg+3 of an n-tile for row lr of an
+  // m-tile: 16 contiguous bytes of the partial row
+  float* out = part + (int64_t)split * rows * n;
+  __syncthreads();  // the ring is drained: its LDS holds the waves' sums
+  f32x4* red = reinterpret_cast<f32x4*>(smem_raw);  // [wave][tile][lane]
 #pragma unroll
-      for (int q = 1; q < 4; ++q) v += red[(q * NJ * MT + tile) * 64 + lane];
-      store(tile / MT, tile % MT, v);
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) red[(wave * NJ * MT + j * MT + i) * 64 + lane] = acc[j][i];
+  __syncthreads();
+  for (int tile = wave; tile < NJ * MT; tile += 4) {
+    f32x4 v = red[tile * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) v += red[(q * NJ * MT + tile) * 64 + lane];
+    const int j = tile / MT, m = 16 * (tile % MT) + lr;
+    if (m < rows) *reinterpret_cast<f32x4*>(out + (int64_t)m * n + n0 + 16 * j + 4 * lg) = v;
+  }
+}
+
+// ---- large column tiles and the gated projection ---------------------------
+//
+// kProducers waves bring the unit's W rows and x through LDS and do nothing
+// else; NW x MW x KG consumer waves compute.  Work goes in k blocks of KS: an
+// x slab (16 MT rows x KS) and SUB = TN / RS steps, each a slot of RS weight
+// rows x KS; a block's slab is issued with its first step.  With KS = 256 an
+// instruction brings 512-byte runs of two rows: the W stream of the Qwen3-8B
+// up/gate alone takes 33.8 us in 512-byte runs, 37.9 in 256-byte runs and
+// 34.3 in 1 KB runs, whatever the depth (48 to 144 KB in flight per CU), so
+// the ring is three slots and the LDS goes to x.  The x slabs cost the stream
+// under 2 us: the same x loaded to registers by the consumers, 64-byte runs of
+// 16 rows, cost 12.  Consumer (ng, mg, kg) takes the slot's tiles ng, ng + NW,
+// ..., the row tiles mg, mg + MW, ... and the kg-th of KG parts of the block's
+// k, with its x operands kept in registers over the block's steps where they
+// fit; only KG > 1 (one unit tile and few rows) needs a sum across waves.
+//
+// Step s may be issued once the consumers have passed the barrier of step
+// s - R + 1, that is once they are done with step s - R, and with the slab of
+// the block XD before when that one's last step is no later: R - 1 <= (XD -
+// 1) SUB.
+constexpr int kProducers = 4;
+
+template <int MT_, int TN_, int RS_, int KS_, int R_, int XD_, int NW_, int MW_, int KG_, bool GATED_>
+struct StreamShape {
+  static constexpr int MT = MT_, TN = TN_, RS = RS_, KS = KS_, R = R_, XD = XD_, NW = NW_, MW = MW_, KG = KG_;
+  static constexpr bool GATED = GATED_;
+  static constexpr int NC = NW * MW * KG, NJ = TN / 16, SUB = TN / RS, JS = RS / 16;
+  static constexpr int kRowB = KS * 2, kSlot = RS * kRowB, kSlab = 16 * MT * kRowB;
+  static constexpr int WI = kSlot / 1024 / kProducers, XI = kSlab / 1024 / kProducers;  // instructions per producer
+  static constexpr int RPI = 1024 / kRowB;                                              // rows per instruction
+  static constexpr int KW = KS / 32 / KG, JW = JS / NW, MI = (MT + MW - 1) / MW;
+  static constexpr bool HOIST = SUB > 1 && KW * MI <= 16;  // a block's x operands in at most 64 registers
+  static constexpr int kThreads = (kProducers + NC) * kWave;
+  static constexpr int kLds = R * kSlot + XD * kSlab;
+  static_assert(WI * kProducers * 1024 == kSlot && XI * kProducers * 1024 == kSlab && JW * NW == JS && SUB * RS == TN);
+  static_assert(R >= 2 && R - 1 <= (XD - 1) * SUB && kLds <= kGemmLds);
+  static_assert(!GATED || (SUB * JW) % 2 == 0);
+  static_assert(KG == 1 || NC * SUB * JW * MI * 1024 <= kLds);
+};
+
+// Unit u as in linear_partials_kernel, in blocks of KS k.
+template <class S>
+__global__ __launch_bounds__(S::kThreads) void stream_gemm_kernel(const f16* __restrict__ x,
+                                                                  const f16* __restrict__ w,
+                                                                  float* __restrict__ part, int rows, int n, int k,
+                                                                  int splits, int n_tiles, f16* __restrict__ y) {
+  constexpr int MT = S::MT, TN = S::TN, RS = S::RS, KS = S::KS, R = S::R, XD = S::XD, P = kProducers;
+  constexpr int SUB = S::SUB, WI = S::WI, XI = S::XI, RPI = S::RPI, KW = S::KW, JW = S::JW, MI = S::MI;
+  extern __shared__ __align__(16) char smem_raw[];
+  lds_char* slabs = (lds_char*)smem_raw;
+  lds_char* ring = slabs + XD * S::kSlab;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nt = blockIdx.x % n_tiles, split = blockIdx.x / n_tiles;
+  const int n0 = nt * (S::GATED ? TN / 2 : TN);
+  const int T = k / KS;
+  const int t0 = (int)((int64_t)split * T / splits);
+  const int blocks = (int)((int64_t)(split + 1) * T / splits) - t0;
+  const int steps = blocks * SUB;
+
+  if (wave < P) {
+    // instruction i of this wave brings rows RPI (P i + wave) .. of a slot or
+    // slab; a lane the 16-byte chunk q ^ (row % 16) of its row
+    const int sub_row = lane / (kWave / RPI), q = lane % (kWave / RPI);
+    const f16* xsrc[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const int r = (i * P + wave) * RPI + sub_row;
+      xsrc[i] = x + (int64_t)(r < rows ? r : rows - 1) * k + (int64_t)t0 * KS + (q ^ chunk_swizzle(r)) * 8;
+    }
+    const f16* wsrc[SUB * WI];
+#pragma unroll
+    for (int i = 0; i < SUB * WI; ++i) {
+      const int r = ((i % WI) * P + wave) * RPI + sub_row;
+      const int row = (i / WI) * RS + r;  // the unit's row: gated, its up rows and then the gate rows, n further on
+      const int wrow = !S::GATED || row < TN / 2 ? n0 + row : n + n0 + row - TN / 2;
+      wsrc[i] = w + (int64_t)wrow * k + (int64_t)t0 * KS + (q ^ chunk_swizzle(r)) * 8;
+    }
+    int slot_no = 0;
+    auto issue = [&](int blk, auto subc) __attribute__((always_inline)) {
+      constexpr int sub = decltype(subc)::value;
+      if constexpr (sub == 0) {
+        const uint32_t slab = (uint32_t)(uintptr_t)(slabs + (blk % XD) * S::kSlab);
+#pragma unroll
+        for (int i = 0; i < XI; ++i) gemm_dma<false>(slab + (i * P + wave) * 1024, xsrc[i] + (int64_t)blk * KS);
+      }
+      const uint32_t slot = (uint32_t)(uintptr_t)(ring + slot_no * S::kSlot);
+      slot_no = slot_no + 1 == R ? 0 : slot_no + 1;
+#pragma unroll
+      for (int i = 0; i < WI; ++i)
+        gemm_dma<true>(slot + (i * P + wave) * 1024, wsrc[sub * WI + i] + (int64_t)blk * KS);
+    };
+    auto issue_step = [&](int s) __attribute__((always_inline)) {
+      const int blk = s / SUB, sub = s - blk * SUB;
+      static_for<SUB>([&](auto u) {
+        if (sub == decltype(u)::value) issue(blk, u);
+      });
+    };
+    int issued = 0;
+    while (issued < R - 1 && issued < steps) issue_step(issued++);
+    for (int s0 = 0; s0 < steps; s0 += SUB) {
+      static_for<SUB>([&](auto u) {
+        constexpr int sub = decltype(u)::value;
+        // this wave's instructions of the R - 2 steps after this one may be
+        // outstanding (their slabs among them); then every producer's step
+        // has landed and the slot of the step before is free
+        constexpr int newer = (R - 2) * WI + (sub + R - 2) / SUB * XI;
+        static_assert(newer <= 63, "vmcnt range");
+        if (issued - (s0 + sub) - 1 >= R - 2) gemm_wait<newer>();
+        else gemm_wait<0>();
+        gemm_barrier();
+        if (issued < steps) issue_step(issued++);
+      });
+    }
+    if constexpr (S::KG > 1) {  // the consumers' two barriers
+      __syncthreads();
+      __syncthreads();
+    }
+    return;
+  }
+
+  const int c = wave - P;
+  const int ng = c % S::NW, mg = c / S::NW % S::MW, kg = c / (S::NW * S::MW);
+  int xrow[MI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int t = i * S::MW + mg;  // past the row tiles: the last one again, not stored
+    xrow[i] = (16 * (t < MT ? t : MT - 1) + lr) * S::kRowB;
+  }
+  f32x4 acc[SUB * JW][MI];
+#pragma unroll
+  for (int j = 0; j < SUB * JW; ++j)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int slot_no = 0;
+  for (int blk = 0; blk < blocks; ++blk) {
+    const lds_char* slab = slabs + (blk % XD) * S::kSlab;
+    f16x8 kept[S::HOIST ? KW : 1][MI];
+#pragma unroll
+    for (int sub = 0; sub < SUB; ++sub) {
+      // this wave's reads of the step before are done, then the step is in
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      const lds_char* sl = ring + slot_no * S::kSlot;
+      slot_no = slot_no + 1 == R ? 0 : slot_no + 1;
+#pragma unroll
+      for (int s = 0; s < KW; ++s) {
+        const int ch = (((kg * KW + s) * 4 + lg) ^ lr) << 4;
+        f16x8 a[JW], b[MI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+          if (S::HOIST && sub > 0) b[i] = kept[S::HOIST ? s : 0][i];
+          else b[i] = *(const lds_f16x8*)(slab + xrow[i] + ch);
+          if (S::HOIST && sub == 0) kept[S::HOIST ? s : 0][i] = b[i];
+        }
+#pragma unroll
+        for (int j = 0; j < JW; ++j) a[j] = *(const lds_f16x8*)(sl + (16 * (ng + j * S::NW) + lr) * S::kRowB + ch);
+#pragma unroll
+        for (int j = 0; j < JW; ++j)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[sub * JW + j][i] = mfma_k32(a[j], b[i], acc[sub * JW + j][i]);
+      }
+    }
+  }
+
+  // lane (lg, lr) holds columns 4lg .. 4lg+3 of a tile for row lr of a row
+  // tile.  Accumulator j is tile ng + (j % JW) NW of step j / JW; gated, the
+  // first half are up tiles and the second their gate tiles.
+  auto column = [&](int j) { return j / JW * RS + 16 * (ng + j % JW * S::NW) + 4 * lg; };
+  auto store = [&](int j, int i, f32x4 v, f32x4 gate) {
+    const int t = i * S::MW + mg, m = 16 * t + lr;
+    if (t >= MT || m >= rows) return;
+    if constexpr (S::GATED) {
+      // the SiLU-and-mul of silu_and_mul_kernel on the fp16-rounded sums
+      f16x4 h;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f16 up = (f16)v[e];
+        const float gf = (float)(f16)gate[e];
+        const f16 sg = (f16)(gf / (1.f + expf(-gf)));
+        h[e] = (f16)((float)up * (float)sg);
+      }
+      *reinterpret_cast<f16x4*>(y + (int64_t)m * n + n0 + column(j)) = h;
+    } else {
+      *reinterpret_cast<f32x4*>(part + ((int64_t)split * rows + m) * n + n0 + column(j)) = v;
+    }
+  };
+  constexpr int NT = SUB * JW, OUT = S::GATED ? NT / 2 : NT;  // accumulator tiles, of which stored
+  if constexpr (S::KG == 1) {
+#pragma unroll
+    for (int j = 0; j < OUT; ++j)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) store(j, i, acc[j][i], acc[S::GATED ? j + OUT : j][i]);
+  } else {
+    // the KG waves of a group add their sums in LDS, in kg order
+    constexpr int TW = NT * MI;
+    f32x4* red = reinterpret_cast<f32x4*>(smem_raw) + c % (S::NW * S::MW) * S::KG * TW * kWave;
+    __syncthreads();  // every wave is past its last slot
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MI; ++i) red[(kg * TW + j * MI + i) * kWave + lane] = acc[j][i];
+    __syncthreads();
+    auto sum = [&](int t) {
+      f32x4 v = red[t * kWave + lane];
+#pragma unroll
+      for (int q = 1; q < S::KG; ++q) v += red[(q * TW + t) * kWave + lane];
+      return v;
+    };
+#pragma unroll
+    for (int u = 0; u < (OUT * MI + S::KG - 1) / S::KG; ++u) {
+      const int t = u * S::KG + kg;
+      if (t < OUT * MI) store(t / MI, t % MI, sum(t), S::GATED ? sum(t + OUT * MI) : f32x4{});
     }
   }
 }
@@ -304,54 +475,97 @@ int check_linear(int64_t n_rows, int64_t n_out, int64_t n_in, const char* who) {
   return NSD_OK;
 }
 
+// Raises a kernel's dynamic-LDS limit once per process: a function-local
+// static is initialised exactly once even when several threads launch at
+// once, and a failure stays reported on every later call.
+template <auto Kernel, int kLds>
+int allow_lds() {
+  static const hipError_t attr =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  return attr == hipSuccess ? NSD_OK : fail(NSD_ERR_HIP, "linear: LDS attribute: %s", hipGetErrorString(attr));
+}
+
+struct GemmArgs {
+  const f16* x;
+  const f16* w;
+  float* part;  // partials, or
+  f16* y;       // the gated output
+  int rows, n, k, splits;
+  hipStream_t st;
+};
+
+template <class S>
+int launch_stream(const GemmArgs& g) {
+  if (int rc = allow_lds<&stream_gemm_kernel<S>, S::kLds>()) return rc;
+  const int n_tiles = g.n / (S::GATED ? S::TN / 2 : S::TN);
+  hipLaunchKernelGGL(stream_gemm_kernel<S>, dim3(n_tiles * g.splits), dim3(S::kThreads), S::kLds, g.st, g.x, g.w,
+                     g.part, g.rows, g.n, g.k, g.splits, n_tiles, g.y);
+  return launch_status(S::GATED ? "up_gate_silu_and_mul" : "linear");
+}
+
 template <int MT, int TN>
-int launch_linear(const f16* x, const f16* w, float* part, int rows, int n, int k, int splits, hipStream_t st) {
-  using S = LinearShape<MT, TN>;
-  // raise the dynamic-LDS limit once per process: a function-local static is
-  // initialised exactly once even when several threads launch at once, and
-  // a failure stays reported on every later call
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&linear_partials_kernel<MT, TN>), hipFuncAttributeMaxDynamicSharedMemorySize,
-      S::kLds);
-  if (attr != hipSuccess) return fail(NSD_ERR_HIP, "linear: LDS attribute: %s", hipGetErrorString(attr));
-  const int n_tiles = n / TN;
-  hipLaunchKernelGGL((linear_partials_kernel<MT, TN>), dim3(n_tiles * splits), dim3(kGemmThreads), S::kLds, st, x,
-                     w, part, rows, n, k, splits, n_tiles, nullptr);
-  return launch_status("linear");
+int launch_linear(const GemmArgs& g) {
+  constexpr int MW = MT > 1 ? 2 : 1, NW = MT > 1 ? 2 : 4;  // one row tile: the waves split the columns
+  if constexpr (TN == 64) {
+    return launch_stream<StreamShape<MT, 64, 64, 128, 3, 3, NW, MW, 1, false>>(g);
+  } else if constexpr (TN == 128) {
+    return launch_stream<StreamShape<MT, 128, 64, 128, 4, 3, NW, MW, 1, false>>(g);
+  } else {
+    using S = LinearShape<MT, TN>;
+    if (int rc = allow_lds<&linear_partials_kernel<MT, TN>, S::kLds>()) return rc;
+    const int n_tiles = g.n / TN;
+    hipLaunchKernelGGL((linear_partials_kernel<MT, TN>), dim3(n_tiles * g.splits), dim3(kGemmThreads), S::kLds, g.st,
+                       g.x, g.w, g.part, g.rows, g.n, g.k, g.splits, n_tiles);
+    return launch_status("linear");
+  }
 }
 
-// The gated (up/gate + SiLU-and-mul) unit: 48 up and 48 gate columns over
-// all of k, one unit per 48 output columns.
-constexpr int kGatedTile = 96;
-constexpr int kGatedMaxRowTiles = 7;  // three ring slots fit up to 112 rows (128 rows: the ring kernel, 1.5 us faster)
-
-template <int MT>
-int launch_gated(const f16* x, const f16* w, f16* y, int rows, int inter, int hidden, hipStream_t st) {
-  using S = LinearShape<MT, kGatedTile, true>;
-  static const hipError_t attr = hipFuncSetAttribute(  // once per process, as in launch_linear
-      reinterpret_cast<const void*>(&linear_partials_kernel<MT, kGatedTile, true>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
-  if (attr != hipSuccess) return fail(NSD_ERR_HIP, "up_gate: LDS attribute: %s", hipGetErrorString(attr));
-  const int n_tiles = inter / (kGatedTile / 2);
-  hipLaunchKernelGGL((linear_partials_kernel<MT, kGatedTile, true>), dim3(n_tiles), dim3(kGemmThreads), S::kLds, st,
-                     x, w, nullptr, rows, inter, hidden, 1, n_tiles, y);
-  return launch_status("up_gate_silu_and_mul");
+// A gated unit of PAIRS up tiles and their gate tiles.  k blocks of 256 while
+// the x slabs leave room for three slots (up to 80 rows) and k allows, else
+// of 128.
+template <int MT, int PAIRS>
+int launch_gated(const GemmArgs& g) {
+  constexpr int TN = 32 * PAIRS;
+  constexpr int MW = MT > 1 ? 2 : 1;
+  if constexpr (PAIRS == 1) {
+    // one slot holds the pair; the waves split the row tiles, or k at one or
+    // two of them
+    constexpr int W = MT >= 3 ? 4 : MT, KG = 4 / W;
+    if constexpr (MT <= 4)
+      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, 32, 256, 3, 3, 1, W, KG, true>>(g);
+    return launch_stream<StreamShape<MT, TN, 32, 128, 4, 4, 1, W, KG, true>>(g);
+  } else {
+    constexpr int RS = PAIRS == 3 ? 48 : 32, NW = RS / 16;
+    if constexpr (MT <= 5)
+      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, RS, 256, 3, 2, NW, MW, 1, true>>(g);
+    return launch_stream<StreamShape<MT, TN, RS, 128, 4, 3, NW, MW, 1, true>>(g);
+  }
 }
 
-template <int... I>
-int launch_gated_rows(std::integer_sequence<int, I...>, int mt, const f16* x, const f16* w, f16* y, int rows,
-                      int inter, int hidden, hipStream_t st) {
+// Calls f<MT>() for the row tiles' count mt in 1 .. kMaxRowTiles.
+template <class F, int... I>
+int with_row_tiles(std::integer_sequence<int, I...>, int mt, F&& f) {
   int rc = NSD_ERR_UNSUPPORTED;
-  ((mt == I + 1 ? (rc = launch_gated<I + 1>(x, w, y, rows, inter, hidden, st), 0) : 0), ...);
+  ((mt == I + 1 ? (rc = f(std::integral_constant<int, I + 1>{}), 0) : 0), ...);
   return rc;
 }
+template <class F>
+int with_row_tiles(int rows, F&& f) {
+  return with_row_tiles(std::make_integer_sequence<int, kMaxRowTiles>{}, (rows + 15) / 16, f);
+}
 
-template <int TN, int... I>
-int launch_linear_rows(std::integer_sequence<int, I...>, int mt, const f16* x, const f16* w, float* part, int rows,
-                       int n, int k, int splits, hipStream_t st) {
-  int rc = NSD_ERR_UNSUPPORTED;
-  ((mt == I + 1 ? (rc = launch_linear<I + 1, TN>(x, w, part, rows, n, k, splits, st), 0) : 0), ...);
-  return rc;
+// Up/gate tile pairs per gated unit, or 0 for a shape the ring kernel takes:
+// the most units (the fewest pairs) that one round of the compute units
+// holds.  At seven tenths of them busy the stream still fills the memory
+// (Qwen3-0.6B, 192 units of 256: 6.2 us against 9.8); below that the ring
+// kernel's balanced ranges, which use every compute unit, are left to it.
+int gated_pairs(int64_t inter, int cus) {
+  for (int pairs = 1; pairs <= 4; ++pairs) {
+    if (inter % (16 * pairs)) continue;
+    const int64_t units = inter / (16 * pairs);
+    if (units <= cus) return units * 10 >= cus * 7 ? pairs : 0;
+  }
+  return 0;
 }
 
 }  // namespace
@@ -361,16 +575,20 @@ int up_gate_silu_gated(const void* x, const void* up_gate, void* y, int64_t n_ro
   *served = false;
   int cus = 0;
   if (int rc = device_cus(&cus)) return rc;
-  const int64_t units = inter / (kGatedTile / 2);
-  // one unit per CU or close to it (fewer units leave CUs idle: the older
-  // kernel spreads small shapes better)
-  if (inter % (kGatedTile / 2) || units * 10 < cus * 9 || units > cus || n_rows > 16 * kGatedMaxRowTiles ||
-      hidden % kKStep)
-    return NSD_OK;
+  const int pairs = gated_pairs(inter, cus);
+  if (pairs == 0 || n_rows > 16 * kMaxRowTiles || hidden % kKStep) return NSD_OK;
   *served = true;
-  return launch_gated_rows(std::make_integer_sequence<int, kGatedMaxRowTiles>{}, (int)((n_rows + 15) / 16),
-                           static_cast<const f16*>(x), static_cast<const f16*>(up_gate), static_cast<f16*>(y),
-                           (int)n_rows, (int)inter, (int)hidden, as_stream(stream));
+  const GemmArgs g{static_cast<const f16*>(x), static_cast<const f16*>(up_gate), nullptr, static_cast<f16*>(y),
+                   (int)n_rows, (int)inter, (int)hidden, 1, as_stream(stream)};
+  return with_row_tiles(g.rows, [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    switch (pairs) {
+      case 1: return launch_gated<MT, 1>(g);
+      case 2: return launch_gated<MT, 2>(g);
+      case 3: return launch_gated<MT, 3>(g);
+      default: return launch_gated<MT, 4>(g);
+    }
+  });
 }
 
 }  // namespace nsd
@@ -395,18 +613,17 @@ extern "C" int nsd_linear_partials(const void* x, const void* w, float* partials
   int cus = 0;
   if (int rc = device_cus(&cus)) return rc;
   const LinearConfig c = choose_linear(n_out, n_in, cus);
-  const int mt = (int)((n_rows + 15) / 16);
-  const auto* xp = static_cast<const f16*>(x);
-  const auto* wp = static_cast<const f16*>(w);
-  const hipStream_t st = as_stream(stream);
-  const auto seq = std::make_integer_sequence<int, kMaxRowTiles>{};
-  const int rows = (int)n_rows, n = (int)n_out, k = (int)n_in;
-  switch (c.tn) {
-    case 16: return launch_linear_rows<16>(seq, mt, xp, wp, partials, rows, n, k, c.splits, st);
-    case 32: return launch_linear_rows<32>(seq, mt, xp, wp, partials, rows, n, k, c.splits, st);
-    case 64: return launch_linear_rows<64>(seq, mt, xp, wp, partials, rows, n, k, c.splits, st);
-    default: return launch_linear_rows<128>(seq, mt, xp, wp, partials, rows, n, k, c.splits, st);
-  }
+  const GemmArgs g{static_cast<const f16*>(x), static_cast<const f16*>(w), partials, nullptr, (int)n_rows, (int)n_out,
+                   (int)n_in, c.splits, as_stream(stream)};
+  return with_row_tiles(g.rows, [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    switch (c.tn) {
+      case 16: return launch_linear<MT, 16>(g);
+      case 32: return launch_linear<MT, 32>(g);
+      case 64: return launch_linear<MT, 64>(g);
+      default: return launch_linear<MT, 128>(g);
+    }
+  });
 }
 
 extern "C" int nsd_sum_partials(const float* partials, int splits, void* y, int64_t n_rows, int64_t n_out,

@@ -28,7 +28,8 @@ from nebulasd_amd import _lib
 from nebulasd_amd.config import QWEN3_0_6B, QWEN3_8B, EngineConfig, ModelConfig
 from nebulasd_amd.infer_state import build_infer_state, rope_cache
 from nebulasd_amd.kernels import (fused_add_rmsnorm_inplace, fused_add_rmsnorm_partials, linear, linear_partials,
-                                  linear_splits, qk_norm_rope_store, qk_norm_rope_store_partials, sum_partials)
+                                  linear_splits, qk_norm_rope_store, qk_norm_rope_store_partials, sum_partials,
+                                  up_gate_silu_and_mul)
 from nebulasd_amd.workload import make_workload
 
 pytestmark = pytest.mark.gpu
@@ -73,6 +74,41 @@ def test_linear_matches_oracle(gpu, rows, n, k):
     assert torch.equal(linear(x, w), y)
     print(f"  {splits} splits; exact vs oracle {exact:.4f}, vs F.linear {float(np.mean(got == lib)):.4f}",
           flush=True)
+
+
+ROW_EDGES = [1, 16, 17, 33, 48, 64, 65, 80, 81, 97, 113, 128]  # both sides of every row-tile count's layout
+
+
+@pytest.mark.parametrize("rows", ROW_EDGES)
+@pytest.mark.parametrize("n,k", [(16384, 128), (16384, 384), (6144, 2688)], ids=["64-1block", "64-3blocks", "128-5splits"])
+def test_linear_row_tiles(gpu, rows, n, k):
+    """The large column tiles at every row-tile count: one k block, an odd count, and uneven splits.
+    fp32 sums of k products of |x w| ~ 0.03 each: within 1e-5 relative plus the same of the rms sum."""
+    x = _randn(gpu, rows, k, seed=31)
+    w = _randn(gpu, n, k, seed=32, scale=0.03)
+    splits = linear_splits(rows, n, k)
+    buf = torch.full((splits * rows * n + n,), 7.0, dtype=torch.float32, device=gpu)
+    got = linear_partials(x, w, buf[:splits * rows * n].view(splits, rows, n)).double().sum(0)
+    assert bool((buf[splits * rows * n:] == 7.0).all()), "the kernel wrote past the partials"
+    want = x.double() @ w.double().t().contiguous()
+    assert ((got - want).abs() <= 1e-5 * want.abs() + 1e-5 * 0.03 * k ** 0.5).all()
+
+
+@pytest.mark.parametrize("rows", ROW_EDGES)
+@pytest.mark.parametrize("inter,hidden", [(3200, 256), (3200, 384), (6144, 512), (6144, 128), (12288, 768),
+                                          (12288, 384), (12800, 512), (12800, 384)])
+def test_gated_row_tiles(gpu, rows, inter, hidden):
+    """The gated units of one to four tile pairs, k blocks of 256 and of 128, at every row-tile count:
+    against float64 with the two fp16 GEMM roundings, the sigmoid's and the product's (2^-11 each, and
+    the gate's error times the SiLU's slope: 2e-3 in all), rows past the output untouched."""
+    x = _randn(gpu, rows, hidden, seed=33)
+    w = _randn(gpu, 2 * inter, hidden, seed=34, scale=hidden ** -0.5)
+    buf = torch.full((rows * inter + inter,), 7.0, dtype=torch.float16, device=gpu)
+    out = up_gate_silu_and_mul(x, w, out=buf[:rows * inter].view(rows, inter))
+    assert bool((buf[rows * inter:] == 7.0).all()), "the kernel wrote past the output"
+    up, gate = (x.double() @ w.double().t().contiguous()).chunk(2, 1)
+    want = up * F.silu(gate)
+    assert ((out.double() - want).abs() <= 2e-3 * want.abs() + 1e-3).all()
 
 
 def test_linear_rejects_bad_shapes(gpu):
