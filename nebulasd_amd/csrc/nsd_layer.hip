@@ -15,7 +15,7 @@
 // The element-wise kernels are HBM-bound (one read and one write of every
 // element) and latency-bound at decode sizes.  lm_head + argmax is a skinny
 // GEMM: the [vocab, hidden] weight (1.24 GB for Qwen3-8B) is streamed once per
-// pass of at most 128 rows of x through an LDS ring by 16x16x32 MFMAs; each
+// pass of at most 128 rows of x through LDS slots by 16x16x32 MFMAs; each
 // wave folds its logits into one 64-bit key per row, (ordered fp16 value <<
 // 32) | ~index, merged with atomicMax so the largest value and then the
 // smallest index win.
@@ -162,54 +162,19 @@ argmax_rows_kernel(const f16* __restrict__ logits, int64_t vocab, int64_t* token
   }
 }
 
-// ---- lm_head GEMV + argmax -----------------------------------------------
-
-constexpr int kLmK = 128;  // hidden must be a multiple of this (one ring step of k)
-
-// lm_head GEMV + argmax through an LDS ring (1..128 rows of x per pass).
+// ---- weight streams through LDS -------------------------------------------
 //
-// One workgroup per CU streams a balanced range of 16-row vocab tiles, in
-// groups of eight tiles (128 vocab rows), in k steps of 128 (256 bytes of a
-// row).  Four producer waves bring each step's weight chunk (128 rows x
-// 256 B) from memory straight into a slot of a kRgRing-slot LDS ring by
-// global_load_lds_dwordx4, four rows x 256 B per instruction: whole 256-byte
-// runs of a row per instruction, against the 64-byte pieces of 16 rows that
-// a 16x16 MFMA operand loaded into registers gets (measured read rates over
-// the Qwen3-8B lm_head: 5.9 against 5.1 TB/s), with kRgRing - 1 steps in
-// flight.  The 16-byte chunk q of slot row r sits at chunk q ^ (r & 15), so
-// the sixteen rows an operand read touches hit distinct banks.  Consumer
-// wave (rt, h) holds x row tile rt in registers (its own loads, three steps
-// ahead; x is a few hundred KB and stays in L2), multiplies it by vocab
-// tiles [h*TPW, (h+1)*TPW) of the group (A = weight rows, B = x rows, as in
-// the register-staged kernel, so every sum runs in the same k order), folds
-// its logits into one running key per x row at the end of each group, and
-// merges it with one atomicMax at the end.  The two roles never wait on
-// each other's loads: each wave's vmcnt counts its own kind only.
-// Out-of-range weight rows are fetched from one fixed row (an L2 hit) and
-// never used.  Measured on MI355X, Qwen3-8B lm_head: 243 us at 1 row and
-// 253 us at 80 (against 266 / 323 for the register-staged kernel).
-constexpr int kRgTiles = 8;                             // vocab tiles per group
-constexpr int kRgRowBytes = 256;                        // a row's 128 k of one step
-constexpr int kRgRing = 4;                              // ring slots: three steps in flight
-constexpr int kRgSlot = kRgTiles * 16 * kRgRowBytes;    // 32 KB
-constexpr int kRgLds = kRgRing * kRgSlot;
+// Shared by lm_head + argmax and the up/gate ring kernel: producer waves that
+// bring weight rows straight from memory into LDS slots with
+// global_load_lds_dwordx4 and do nothing else.
+constexpr int kLmK = 128;           // hidden must be a multiple of this
+constexpr int kRgRowBytes = 256;    // a row's 128 k of one step (up/gate ring)
 constexpr int kRgProducers = 4;
-constexpr int kRgInsPerWave = kRgTiles * 16 / 4 / kRgProducers;  // DMA instructions per producer per step
-constexpr int kRgXAhead = 3;                            // steps of x a consumer loads ahead
-constexpr int kRgMaxRowTiles = 8;                       // up to 128 rows of x per pass
-static_assert(kRgLds <= 160 * 1024, "ring fits the CU's LDS");
-static_assert(kRgInsPerWave * (kRgRing - 1) <= 63, "vmcnt range");
+constexpr int kRgMaxRowTiles = 8;   // up to 128 rows of x per pass
 
-// Consumer waves per x row tile: 8, 4, then 1 for 3..8 row tiles (a second
-// wave per tile would load the tile's x again: measured slower at 64-80 rows).
-template <int NRT>
-constexpr int rg_split() { return NRT == 1 ? 8 : NRT == 2 ? 4 : 1; }
-template <int NRT>
-constexpr int rg_threads() { return (kRgProducers + NRT * rg_split<NRT>()) * kWave; }
-
-// A weight chunk into a ring slot.  NT: non-temporal, for the pass that reads
-// the weight last.  A model's weights pass through the caches once a forward,
-// so keeping them out of the replacement costs nothing and the stream runs
+// A weight chunk into a slot.  NT: non-temporal, for the pass that reads the
+// weight last.  A model's weights pass through the caches once a forward, so
+// keeping them out of the replacement costs nothing and the stream runs
 // faster: lm_head 151936 x 4096, 80 rows 236 -> 225 us.  Earlier passes of a
 // call with more than 128 rows keep the default policy: the next pass reads
 // the same weight again.
@@ -227,144 +192,226 @@ template <int N>
 __device__ inline void rg_wait_n() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
-// A producer's loads of all but its n most recent steps are complete
-// (0 <= n <= kRgRing - 2).
-template <int N>
-__device__ inline void rg_wait_steps_n() {
-  if constexpr (N * kRgInsPerWave <= 63) rg_wait_n<N * kRgInsPerWave>();
-  else rg_wait_n<0>();
-}
-__device__ inline void rg_wait_steps(int n) {
-  static_assert(kRgRing <= 6, "wait table");
-  switch (n) {
-    case 1: rg_wait_steps_n<1>(); break;
-    case 2: rg_wait_steps_n<2>(); break;
-    case 3: rg_wait_steps_n<3>(); break;
-    case 4: rg_wait_steps_n<4>(); break;
-    default: rg_wait_n<0>(); break;
-  }
-}
 
-template <int NRT>
-__global__ void __launch_bounds__(rg_threads<NRT>())
-lm_ring_kernel(const f16* __restrict__ x, const f16* __restrict__ w, int n_rows, int hidden, int64_t vocab,
-               uint64_t* __restrict__ keys, bool last_pass) {
-  constexpr int SPLIT = rg_split<NRT>(), TPW = kRgTiles / SPLIT, XR = kRgXAhead + 1;
+// ---- lm_head GEMV + argmax -----------------------------------------------
+//
+// One workgroup per CU streams a balanced range of 16-row vocab tiles against
+// up to 128 rows of x.  The range goes in `groups` equal groups of `subs`
+// steps of JS tiles (at most kSubs steps), each group over all of k in blocks
+// of KS: a block is an x slab (16 MT rows x KS) and the group's steps, a step
+// one slot of RS weight rows x KS.  Four producer waves bring both; consumer
+// (ng, mg) multiplies row tile mg by the tiles ng, ng + NW, ... of every step
+// (A = weight rows, B = x rows, held in registers over the block's steps) and
+// folds its logits into a running best at the end of a group.
+//
+// Bound by the weight's stream from memory.  131072 x 4096 streamed with no
+// arithmetic takes 170 us, 154 with non-temporal loads (7 TB/s); the rest is
+// x, and the ends.  Groups as large as the accumulators allow re-read x
+// least: two groups of up to 20 tiles at 151936 rows, x a quarter of the
+// weight's bytes through L2.  us per call at 1 / 80 / 128 rows, before (groups
+// of eight tiles, x loaded to registers by every consumer) -> now: 151936 x
+// 4096 237 / 240 / 293 -> 192 / 206 / 234; 151936 x 1024 75 / 70 / 85 -> 52 /
+// 63 / 70; 32000 x 1024 37 / 22 / 25 -> 17 / 20 / 22.  k blocks of 256 (32
+// rows a slot) ran two to five row tiles at 250-364 us, a fifth slot made
+// ranges of two or three steps serial (32000 rows: 59 -> 71) and gained
+// nothing elsewhere.
+//
+// A step may be issued R - 1 steps ahead: its slot is free once the consumers
+// are past the step R before, and its slab (read into registers at a block's
+// first step) once they are past the first step of the block XD = 2 before,
+// which asks for 2 subs >= R.  Ranges of fewer steps than that (a vocabulary
+// of a few tiles per CU) are issued a step at a time.
+template <int MT_>
+struct LmShape {
+  static constexpr int MT = MT_, KS = 128, R = 4, XD = 2;
+  static constexpr int RS = 64;                           // weight rows per step: 16 KB slots
+  static constexpr int JS = RS / 16;                      // tiles per step
+  static constexpr int kSubs = 20 / JS;                   // most steps of a group
+  static constexpr int NW = MT <= 2 ? 2 : 1, MW = MT;     // consumer waves: over the step's tiles, over row tiles
+  static constexpr int JW = JS / NW, KW = KS / 32;
+  static constexpr int kRowB = 2 * KS, kSlot = RS * kRowB, kSlab = 16 * MT * kRowB;
+  static constexpr int RPI = 1024 / kRowB;                // rows per instruction
+  static constexpr int WI = kSlot / 1024 / kRgProducers, XI = kSlab / 1024 / kRgProducers;
+  static constexpr int kThreads = (kRgProducers + NW * MW) * kWave;
+  static constexpr int kKeys = 16 * MT * 8;               // a 64-bit key per row, after the slots
+  static constexpr int kLds = R * kSlot + XD * kSlab + kKeys;
+  static_assert(XI * kRgProducers * 1024 == kSlab && kLds <= 160 * 1024);
+  static_assert((R - 2) * WI + XI <= 63 && 2 * (R - 2) >= R, "waits");
+};
+
+// A lane's running argmax over its logits of one x row, visited in rising
+// vocab order: the fp16-rounded value and its index, the first maximum kept
+// (-0 and +0 are equal, as floats compare), and the first NaN, which is above
+// every value.
+struct LmBest {
+  float v;
+  uint32_t at, nan_at;
+};
+constexpr uint32_t kNoIndex = 0xffffffffu;
+
+template <class S>
+__global__ void __launch_bounds__(S::kThreads)
+lm_stream_kernel(const f16* __restrict__ x, const f16* __restrict__ w, int n_rows, int hidden, int64_t vocab,
+                 uint64_t* __restrict__ keys, int groups, int subs, bool last_pass) {
+  constexpr int MT = S::MT, KS = S::KS, R = S::R, P = kRgProducers, JW = S::JW, KW = S::KW, SUBS = S::kSubs;
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+  lds_char* slabs = (lds_char*)lds_raw;
+  lds_char* ring = slabs + S::XD * S::kSlab;
+  uint64_t* row_keys = reinterpret_cast<uint64_t*>(lds_raw + S::XD * S::kSlab + R * S::kSlot);
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool producer = wv < kRgProducers;
-  const int cw = wv - kRgProducers;  // consumer index
-  const int rt = cw % NRT, h = cw / NRT;
   const int64_t n_tiles = (vocab + 15) / 16;
   const int64_t t0 = (int64_t)blockIdx.x * n_tiles / gridDim.x;
   const int64_t t1 = (int64_t)(blockIdx.x + 1) * n_tiles / gridDim.x;
-  const int kch = hidden / 128;
-  const int steps = (int)((t1 - t0 + kRgTiles - 1) / kRgTiles) * kch;
-  const uint32_t ring = (uint32_t)(uintptr_t)lds_raw;
+  const int kbs = hidden / KS;
+  const int steps = groups * kbs * subs;
+  for (int i = threadIdx.x; i < 16 * MT; i += S::kThreads) row_keys[i] = 0;
+  __syncthreads();
 
-  // Producer wv: instructions j = wv, wv + kRgProducers, ... of step st, slot rows 4j .. 4j+3.
-  auto issue = [&](auto nt, int st) __attribute__((always_inline)) {
-    const int g = st / kch, c = st - g * kch;
-    const uint32_t slot = ring + (uint32_t)((st % kRgRing) * kRgSlot);
+  if (wv < P) {
+    // instruction i of this wave brings rows RPI (P i + wv) .. of a slot or
+    // slab; a lane the 16-byte chunk q ^ (row % 16) of its row.  Weight rows
+    // past the range are fetched from one fixed row (an L2 hit), never used.
+    const int sub_row = lane / (kWave / S::RPI), q = lane % (kWave / S::RPI);
+    const f16* xsrc[S::XI];
 #pragma unroll
-    for (int n = 0; n < kRgInsPerWave; ++n) {
-      const int j = wv + kRgProducers * n;
-      const int r = 4 * j + (lane >> 4);
-      const int64_t tile = t0 + (int64_t)g * kRgTiles + (r >> 4);
-      const int64_t v = tile * 16 + (r & 15);
-      const f16* row = w + (tile < t1 && v < vocab ? v : vocab - 1) * (int64_t)hidden;
-      rg_dma<decltype(nt)::value>(slot + (uint32_t)(4 * j * kRgRowBytes), row + c * 128 + ((lane & 15) ^ (r & 15)) * 8);
+    for (int i = 0; i < S::XI; ++i) {
+      const int r = (i * P + wv) * S::RPI + sub_row;
+      xsrc[i] = x + (int64_t)(r < n_rows ? r : n_rows - 1) * hidden + (q ^ (r & 15)) * 8;
     }
-  };
-  // Consumer: x row tile rt, k = c*128 + 32s + 8*lg .. +7 for s = 0..3 (the B operand of step st).
-  const f16* xrow = x + (int64_t)(rt * 16 + li < n_rows ? rt * 16 + li : n_rows - 1) * hidden + 8 * lg;
-  auto load_x = [&](u32x4 (&xv)[4], int st) __attribute__((always_inline)) {
-    const int c = st % kch;
+    const int64_t v_end = t1 * 16 < vocab ? t1 * 16 : vocab;
+    auto produce = [&](auto nt) __attribute__((always_inline)) {
+      int g = 0, kb = 0, sub = 0, blk = 0, slot_no = 0;  // of the next step to issue
+      auto issue = [&]() __attribute__((always_inline)) {
+        if (sub == 0) {
+          const uint32_t slab = (uint32_t)(uintptr_t)(slabs + (blk & 1) * S::kSlab);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) xv[s] = *reinterpret_cast<const u32x4*>(xrow + c * 128 + 32 * s);
-  };
-
-  auto produce = [&](auto nt) __attribute__((always_inline)) {
-    int issued = 0;
-    while (issued < steps && issued < kRgRing - 1) issue(nt, issued++);
-    for (int i = 0; i < steps; ++i) {
-      rg_wait_steps(issued - i - 1);            // step i landed (this producer's part) ...
-      asm volatile("s_barrier" ::: "memory");   // ... and the other producers'; step i-1's slot is free
-      if (issued < steps) issue(nt, issued++);
-    }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  };
-  if (producer) {
+          for (int i = 0; i < S::XI; ++i) rg_dma<false>(slab + (i * P + wv) * 1024, xsrc[i] + (int64_t)kb * KS);
+        }
+        const uint32_t slot = (uint32_t)(uintptr_t)(ring + slot_no * S::kSlot);
+        const int64_t v0 = (t0 + (int64_t)(g * subs + sub) * S::JS) * 16;
+#pragma unroll
+        for (int i = 0; i < S::WI; ++i) {
+          const int r = (i * P + wv) * S::RPI + sub_row;
+          const f16* row = w + (v0 + r < v_end ? v0 + r : vocab - 1) * (int64_t)hidden;
+          rg_dma<decltype(nt)::value>(slot + (i * P + wv) * 1024, row + (int64_t)kb * KS + (q ^ (r & 15)) * 8);
+        }
+        slot_no = slot_no + 1 == R ? 0 : slot_no + 1;
+        if (++sub == subs) {
+          sub = 0;
+          ++blk;
+          if (++kb == kbs) {
+            kb = 0;
+            ++g;
+          }
+        }
+      };
+      const bool deep = subs >= R - 2;  // else a step at a time
+      const int depth = deep ? R - 1 : 1;
+      int issued = 0;
+      while (issued < depth && issued < steps) {
+        issue();
+        ++issued;
+      }
+      int at = 0;  // the awaited step's place in its block
+      for (int s = 0; s < steps; ++s) {
+        // this wave's part of step s has landed: all but its instructions of
+        // the R - 2 steps after it (one slab among them when the block ends)
+        if (deep && issued - s - 1 >= R - 2) {
+          if (at + R - 2 >= subs) rg_wait_n<(R - 2) * S::WI + S::XI>();
+          else rg_wait_n<(R - 2) * S::WI>();
+        } else {
+          rg_wait_n<0>();
+        }
+        asm volatile("s_barrier" ::: "memory");  // ... and the others'; the slot of step s - 1 is free
+        at = at + 1 == subs ? 0 : at + 1;
+        if (issued < steps) {
+          issue();
+          ++issued;
+        }
+      }
+    };
     if (last_pass) produce(std::true_type{});
     else produce(std::false_type{});
-    return;
-  }
-  // Consumer.  x of step i sits in xv[i % XR].  The main loop runs whole
-  // blocks of XR steps unrolled with no guard, so the register ring keeps
-  // static indices and no register copy waits on a load in flight; every
-  // load is unconditional (steps past the end reload the last step's x).
-  // Steps past the last whole block (only when hidden / 128 is not a
-  // multiple of XR) load their x just before use.
-  f32x4 acc[TPW];
+    __syncthreads();  // the consumers' keys
+  } else {
+    const int c = wv - P, ng = c % S::NW, mg = c / S::NW;
+    const int xrow = (16 * mg + li) * S::kRowB;
+    f32x4 acc[SUBS][JW];
 #pragma unroll
-  for (int a = 0; a < TPW; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-  uint64_t best = 0;  // this lane's largest key over every group so far (a max folds in any order)
-  auto compute = [&](int i, const u32x4 (&xs)[4]) __attribute__((always_inline)) {
-    const lds_char* sl = (const lds_char*)lds_raw + (i % kRgRing) * kRgSlot;
+    for (int u = 0; u < SUBS; ++u)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int q = (4 * s + lg) ^ li;
-      const f16x8 b = as_h8(xs[s]);
+      for (int j = 0; j < JW; ++j) acc[u][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    LmBest best = {-INFINITY, kNoIndex, kNoIndex};
+    int slot_no = 0, blk = 0;
+    for (int g = 0; g < groups; ++g) {
+      for (int kb = 0; kb < kbs; ++kb, ++blk) {
+        const lds_char* slab = slabs + (blk & 1) * S::kSlab;
+        f16x8 b[KW];
 #pragma unroll
-      for (int a = 0; a < TPW; ++a) {
-        const int wr = (h * TPW + a) * 16 + li;
-        acc[a] = mfma_k32(as_h8(*reinterpret_cast<const lds_u32x4*>(sl + wr * kRgRowBytes + q * 16)), b, acc[a]);
-      }
-    }
-    if ((i + 1) % kch == 0) {  // group end: acc[a][e] is vocab row 4*lg + e of tile a, x row rt*16 + li
-      const int64_t tg = t0 + (int64_t)(i / kch) * kRgTiles + h * TPW;
+        for (int u = 0; u < SUBS; ++u) {
+          if (u >= subs) break;
+          // this wave's reads of the step before are done, then the step is in
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          const lds_char* sl = ring + slot_no * S::kSlot;
+          slot_no = slot_no + 1 == R ? 0 : slot_no + 1;
 #pragma unroll
-      for (int a = 0; a < TPW; ++a) {
+          for (int k = 0; k < KW; ++k) {
+            const int ch = ((4 * k + lg) ^ li) << 4;
+            if (u == 0) b[k] = *(const lds_f16x8*)(slab + xrow + ch);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t v = (tg + a) * 16 + 4 * lg + e;
-          if (tg + a < t1 && v < vocab) best = umax64(best, argmax_key((f16)acc[a][e], (uint32_t)v));
+            for (int j = 0; j < JW; ++j)
+              acc[u][j] =
+                  mfma_k32(*(const lds_f16x8*)(sl + (16 * (ng + j * S::NW) + li) * S::kRowB + ch), b[k], acc[u][j]);
+          }
         }
-        acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
+      // acc[u][j][e] is vocab row 4 lg + e of its tile, x row 16 mg + li
+      bool nan = false;
+      auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < SUBS; ++u) {
+          if (u >= subs) break;
+#pragma unroll
+          for (int j = 0; j < JW; ++j) {
+            const int64_t tile = t0 + (int64_t)(g * subs + u) * S::JS + ng + j * S::NW;
+            if (tile >= t1) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int64_t v = tile * 16 + 4 * lg + e;
+              if (v < vocab) f((float)(f16)acc[u][j][e], (uint32_t)v);
+            }
+          }
+        }
+      };
+      each([&](float f, uint32_t v) {
+        // the first value is taken whatever it is (a row of -inf has index 0)
+        const bool up = f > best.v || best.at == kNoIndex;
+        best.v = up ? f : best.v;
+        best.at = up ? v : best.at;
+        nan |= f != f;
+      });
+      if (__any(nan))
+        each([&](float f, uint32_t v) {
+          if (f != f && best.nan_at == kNoIndex) best.nan_at = v;
+        });
+#pragma unroll
+      for (int u = 0; u < SUBS; ++u)
+#pragma unroll
+        for (int j = 0; j < JW; ++j) acc[u][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-  };
-  const int full = steps - steps % XR;
-  u32x4 xv[XR][4];
-  static_for<kRgXAhead>([&](auto u) {
-    constexpr int k = decltype(u)::value;
-    load_x(xv[k], k < steps ? k : steps - 1);
-  });
-  for (int i0 = 0; i0 < full; i0 += XR) {
-    static_for<XR>([&](auto u) {
-      constexpr int k = decltype(u)::value;  // step i0 + k uses xv[k]; xv[(k + kRgXAhead) % XR] is refilled
-      const int i = i0 + k;
-      // the refill is issued before the barrier, which the compiler cannot
-      // move loads across: it cannot sink it next to the loads' first use
-      const int nx = i + kRgXAhead;
-      load_x(xv[(k + kRgXAhead) % XR], nx < steps ? nx : steps - 1);
-      asm volatile("s_barrier" ::: "memory");  // step i's weight chunk is in its slot
-      compute(i, xv[k]);
-    });
+    uint64_t key = 0;
+    if (best.nan_at != kNoIndex) key = argmax_key(__builtin_bit_cast(f16, (uint16_t)0x7e00), best.nan_at);
+    else if (best.at != kNoIndex) key = argmax_key((f16)best.v, best.at);
+    key = umax64(key, shfl_xor64(key, 16));
+    key = umax64(key, shfl_xor64(key, 32));
+    if (lg == 0 && key)
+      atomicMax(reinterpret_cast<unsigned long long*>(row_keys + 16 * mg + li), (unsigned long long)key);
+    __syncthreads();
   }
-  for (int i = full; i < steps; ++i) {
-    asm volatile("s_barrier" ::: "memory");
-    u32x4 xs[4];
-    load_x(xs, i);
-    compute(i, xs);
-  }
-  // One key per x row and wave: the four lane groups' rows, then one atomic.
-  best = umax64(best, shfl_xor64(best, 16));
-  best = umax64(best, shfl_xor64(best, 32));
-  const int row = rt * 16 + li;
-  if (lg == 0 && row < n_rows && best)
-    atomicMax(reinterpret_cast<unsigned long long*>(keys + row), (unsigned long long)best);
+  for (int r = threadIdx.x; r < n_rows; r += S::kThreads)
+    if (row_keys[r])
+      atomicMax(reinterpret_cast<unsigned long long*>(keys + r), (unsigned long long)row_keys[r]);
 }
 
 int rg_grid() {
@@ -378,24 +425,27 @@ int rg_grid() {
   return cus;
 }
 
-template <int NRT>
-void launch_rg(const f16* x, const f16* w, int rows, int hidden, int64_t vocab, uint64_t* keys, bool last_pass,
+template <class S>
+void launch_lm(const f16* x, const f16* w, int rows, int hidden, int64_t vocab, uint64_t* keys, bool last_pass,
                hipStream_t s) {
   static bool attr = [] {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&lm_ring_kernel<NRT>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, kRgLds) == hipSuccess;
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&lm_stream_kernel<S>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds) == hipSuccess;
   }();
   (void)attr;
   const int64_t n_tiles = (vocab + 15) / 16;
-  const unsigned grid = (unsigned)std::min<int64_t>(rg_grid(), n_tiles);
-  hipLaunchKernelGGL(lm_ring_kernel<NRT>, dim3(grid), dim3(rg_threads<NRT>()), kRgLds, s, x, w, rows, hidden, vocab,
-                     keys, last_pass);
+  const int64_t grid = std::min<int64_t>(rg_grid(), n_tiles);
+  const int64_t steps = ((n_tiles + grid - 1) / grid + S::JS - 1) / S::JS;  // of the longest range
+  const int64_t groups = (steps + S::kSubs - 1) / S::kSubs;
+  const int64_t subs = (steps + groups - 1) / groups;
+  hipLaunchKernelGGL(lm_stream_kernel<S>, dim3((unsigned)grid), dim3(S::kThreads), S::kLds, s, x, w, rows, hidden,
+                     vocab, keys, (int)groups, (int)subs, last_pass);
 }
 
 template <int... N>
-void launch_rg_rows(std::integer_sequence<int, N...>, int nrt, const f16* x, const f16* w, int rows, int hidden,
-                    int64_t vocab, uint64_t* keys, bool last_pass, hipStream_t s) {
-  ((nrt == N + 1 ? launch_rg<N + 1>(x, w, rows, hidden, vocab, keys, last_pass, s) : void()), ...);
+void launch_lm_any(std::integer_sequence<int, N...>, int mt, const f16* x, const f16* w, int rows, int hidden,
+                   int64_t vocab, uint64_t* keys, bool last_pass, hipStream_t s) {
+  ((mt == N + 1 ? launch_lm<LmShape<N + 1>>(x, w, rows, hidden, vocab, keys, last_pass, s) : void()), ...);
 }
 
 // ---- up/gate projection + SiLU·mul ----------------------------------------
@@ -664,8 +714,8 @@ extern "C" int nsd_lm_head_argmax(const void* x, const void* lm_head, int64_t n_
     const int rows = (int)std::min<int64_t>(128, n_rows - r0);
     const f16* xr = xp + r0 * hidden;
     uint64_t* kr = keys + r0;
-    launch_rg_rows(std::make_integer_sequence<int, kRgMaxRowTiles>{}, (rows + 15) / 16, xr, wp, rows, (int)hidden,
-                   vocab, kr, r0 + rows == n_rows, s);
+    launch_lm_any(std::make_integer_sequence<int, kRgMaxRowTiles>{}, (rows + 15) / 16, xr, wp, rows, (int)hidden,
+                  vocab, kr, r0 + rows == n_rows, s);
     if (int e = launch_status("lm_head_argmax")) return e;
   }
   hipLaunchKernelGGL(argmax_finalize_kernel, dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, s, keys, tokens,

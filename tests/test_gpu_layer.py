@@ -153,6 +153,40 @@ def test_lm_head_argmax_matches_oracle(gpu, rows, hidden, vocab):
     assert (got.numpy() == want).mean() >= 0.98
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 48, 64, 65, 80, 81, 97, 113, 128])
+@pytest.mark.parametrize("hidden,vocab", [(128, 5), (256, 4096), (384, 8200), (512, 4096 * 20 + 16 * 3), (256, 90001)])
+def test_lm_head_row_tiles_and_ranges(gpu, rows, hidden, vocab):
+    """Every row-tile count with k blocks of 256 and of 128, one to many steps and groups per range, uneven
+    ranges, a last tile that the vocabulary ends in: each row's token is a planted row whose logit stands
+    clear of the rest (|noise logits| stay under 0.5 sqrt(hidden) < hidden / 2), at the range's edges among others."""
+    g = torch.Generator(device=gpu).manual_seed(rows + hidden)
+    w = (torch.rand((vocab, hidden), device=gpu, generator=g) - 0.5).half() * 0.125
+    at = torch.randint(0, vocab, (rows,), device=gpu, generator=g)
+    edges = torch.tensor([0, vocab - 1, vocab // 2], device=gpu)[:rows]
+    at[:edges.numel()] = edges
+    signs = torch.where(torch.rand((rows, hidden), device=gpu, generator=g) < 0.5, -1.0, 1.0)
+    at, first = torch.unique(at, return_inverse=True)
+    w[at] = signs[:at.numel()].half()
+    x = signs[first].half()
+    assert torch.equal(lm_head_argmax(x, w), at[first])
+
+
+def test_lm_head_argmax_special_values(gpu):
+    """All logits -inf: index 0; all equal: index 0; the first of several NaN; -0 before +0 stays first."""
+    hidden, vocab = 256, 20000
+    w = torch.zeros((vocab, hidden), dtype=torch.float16, device=gpu)
+    x = torch.ones((3, hidden), dtype=torch.float16, device=gpu)
+    assert lm_head_argmax(x, w).tolist() == [0, 0, 0]
+    w[:5000] = -0.0
+    assert lm_head_argmax(x, w).tolist() == [0, 0, 0]
+    w[:] = -65504.0
+    assert lm_head_argmax(x, w).tolist() == [0, 0, 0]
+    w[:] = 0.0
+    w[77] = 1.0
+    w[[4097, 19999, 12345]] = float("nan")
+    assert lm_head_argmax(x, w).tolist() == [4097] * 3
+
+
 def test_lm_head_argmax_wide_many_rows(gpu):
     """200 rows (two passes of the fused kernel) at hidden 2048: the fused
     tokens agree with the library GEMM + the argmax kernel and with float64
