@@ -49,6 +49,7 @@
 // Layouts (reference swiftLLM/swiftllm/worker/kernels/paged_attn.py):
 //   k/v cache [N, L, Hkv, 16, 128] fp16, block (blk, layer, head) = 4 KB
 //   contiguous at ((blk*L + layer)*Hkv + head)*16*128 (:49-50, :70-71).
+#include <algorithm>
 #include <mutex>
 
 #include "nsd_device.h"
@@ -211,13 +212,118 @@ __device__ inline void merge_row(const AttnArgs& a, int head, int first, int n_s
   if (d8 == 0 && a.lse != nullptr) a.lse[orow] = (M + __log2f(W)) * kLn2;
 }
 
-// Workgroup (c, g) merges rows 16g .. 16g+15 of combine record c, one thread
-// per (row, 8 dims).
+// Threads per (row, 8 dims) of the merge: one while a segment's slots are one
+// round of a thread's loads (8), else four (up to 32 slots) or sixteen.  The
+// merge is latency-bound, and a round is one more trip to memory: one request
+// of 32k tokens, 64 slots a segment, took 8.1 us with one thread in eight
+// rounds and takes 3.9 with sixteen threads in one; 9 to 17 slots (ragged
+// verify) 4.6 either way.
+constexpr int kMergeSlots = 8;
+
+// A partly merged row: running max (log2), sum of weights, 8 dims.
+struct MergeState {
+  float M, W;
+  f32x4 lo, hi;
+};
+__device__ inline void merge_states(MergeState& a, float M2, float W2, f32x4 lo2, f32x4 hi2) {
+  const float M = fmaxf(a.M, M2);
+  const float use = M == -INFINITY ? 0.f : M;  // neither holds a slot
+  const float s1 = exp2f(a.M - use), s2 = exp2f(M2 - use);
+  a.lo = a.lo * s1 + lo2 * s2;
+  a.hi = a.hi * s1 + hi2 * s2;
+  a.W = a.W * s1 + W2 * s2;
+  a.M = M;
+}
+
+// merge_row for segments of many slots: SL threads take slots sl, sl + SL,
+// ... of a (row, 8 dims) each, and their states are merged over the wave's
+// 16-lane rows and, past four threads, over the workgroup's waves in LDS, in a
+// fixed order.
+template <int SL>
+__device__ inline void merge_row_wide(const AttnArgs& a, int head, int first, int n_slots, int row_start, int n,
+                                      int n_rows, int d8, int sl) {
+  const int nr = n < n_rows ? n : 0;  // every thread takes part in the exchanges
+  const f16* po = a.part_o + ((int64_t)first * a.rows_max + nr) * D + 8 * d8;
+  const float* pl = a.part_lse + (int64_t)first * a.rows_max + nr;
+  MergeState st = {-INFINITY, 0.f, {0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  for (int s0 = sl; s0 < n_slots; s0 += 4 * SL) {
+    float ls[4];
+    f16x8 h[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int s = s0 + SL * u;
+      const int at = s < n_slots ? s : s0;
+      ls[u] = s < n_slots ? pl[(int64_t)at * a.rows_max] : -INFINITY;
+      h[u] = *reinterpret_cast<const f16x8*>(po + (int64_t)at * a.rows_max * D);
+    }
+    const float M = fmaxf(fmaxf(fmaxf(ls[0], ls[1]), fmaxf(ls[2], ls[3])), st.M);
+    const float use = M == -INFINITY ? 0.f : M;
+    const float keep = exp2f(st.M - use);
+    st.lo *= keep;
+    st.hi *= keep;
+    st.W *= keep;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float wgt = exp2f(ls[u] - use);
+      st.lo += f32x4{(float)h[u][0], (float)h[u][1], (float)h[u][2], (float)h[u][3]} * wgt;
+      st.hi += f32x4{(float)h[u][4], (float)h[u][5], (float)h[u][6], (float)h[u][7]} * wgt;
+      st.W += wgt;
+    }
+    st.M = M;
+  }
+#pragma unroll
+  for (int m = 16; m <= 32; m <<= 1) {  // the wave's four 16-lane rows
+    f32x4 lo, hi;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      lo[e] = __shfl_xor(st.lo[e], m, kWave);
+      hi[e] = __shfl_xor(st.hi[e], m, kWave);
+    }
+    const float M2 = __shfl_xor(st.M, m, kWave), W2 = __shfl_xor(st.W, m, kWave);
+    merge_states(st, M2, W2, lo, hi);
+  }
+  if constexpr (SL == 16) {
+    __shared__ MergeState s_wave[4][16];
+    if ((threadIdx.x & 63) < 16) s_wave[threadIdx.x >> 6][d8] = st;
+    __syncthreads();
+    if (threadIdx.x >= 16) return;
+#pragma unroll
+    for (int v = 1; v < 4; ++v) merge_states(st, s_wave[v][d8].M, s_wave[v][d8].W, s_wave[v][d8].lo, s_wave[v][d8].hi);
+  }
+  if (n >= n_rows || sl != 0) return;
+  const float inv = 1.f / st.W;
+  const int qi = n / a.gqa, gh = n - qi * a.gqa;
+  const int64_t orow = (int64_t)(row_start + qi) * a.hq + head * a.gqa + gh;
+  f16x8 hv;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hv[e] = (f16)(st.lo[e] * inv);
+    hv[e + 4] = (f16)(st.hi[e] * inv);
+  }
+  *reinterpret_cast<f16x8*>(a.o + orow * D + 8 * d8) = hv;
+  if (d8 == 0 && a.lse != nullptr) a.lse[orow] = (st.M + __log2f(st.W)) * kLn2;
+}
+
+// Row group `group` of a segment, SL threads per (row, 8 dims): 16 / SL rows
+// a workgroup.
+template <int SL>
+__device__ inline void merge_group(const AttnArgs& a, int head, int first, int n_slots, int row_start, int n_rows,
+                                   int group) {
+  const int d8 = threadIdx.x & 15, p = threadIdx.x >> 4;
+  const int n = group * (16 / SL) + p / SL;
+  if constexpr (SL == 1) {
+    if (n < n_rows) merge_row(a, head, first, n_slots, row_start, n, d8);
+  } else {
+    if (group * (16 / SL) < n_rows) merge_row_wide<SL>(a, head, first, n_slots, row_start, n, n_rows, d8, p % SL);
+  }
+}
+
+// Workgroup (c, g) merges row group g of combine record c.
+template <int SL>
 __global__ __launch_bounds__(256) void combine_kernel(AttnArgs a, int row_groups) {
   const int32_t* c = a.combines + kPieceWords * (blockIdx.x / row_groups);
-  const int n = 16 * (blockIdx.x % row_groups) + (threadIdx.x >> 4);
-  if (n >= c[kCombQLen] * a.gqa) return;
-  merge_row(a, c[kCombHead], c[kCombFirst], c[kCombSlots], c[kCombRowStart], n, threadIdx.x & 15);
+  merge_group<SL>(a, c[kCombHead], c[kCombFirst], c[kCombSlots], c[kCombRowStart], c[kCombQLen] * a.gqa,
+                  blockIdx.x % row_groups);
 }
 
 // The combine records of plans with at most kCombineTableMax of them, packed
@@ -231,12 +337,11 @@ struct CombineTable {
 
 // Workgroup (c, g) = (blockIdx.x, blockIdx.y): the entry's address depends on
 // the workgroup index alone, so it loads with the other arguments.
+template <int SL>
 __global__ __launch_bounds__(256) void combine_table_kernel(AttnArgs a, CombineTable tab) {
   const uint64_t e = tab.e[blockIdx.x];
-  const int n = 16 * (int)blockIdx.y + (threadIdx.x >> 4);
-  if (n >= (int)(e >> 56) * a.gqa) return;
-  merge_row(a, (int)((e >> 28) & 0xff), (int)(e & 0xfffff), (int)((e >> 20) & 0xff), (int)((e >> 36) & 0xfffff), n,
-            threadIdx.x & 15);
+  merge_group<SL>(a, (int)((e >> 28) & 0xff), (int)(e & 0xfffff), (int)((e >> 20) & 0xff), (int)((e >> 36) & 0xfffff),
+                  (int)(e >> 56) * a.gqa, (int)blockIdx.y);
 }
 
 // One workgroup streams one piece: blocks [blk_begin, blk_end) of a (group,
@@ -964,6 +1069,8 @@ int paged_attention_impl(const void* q, void* o, float* lse, const void* k_cache
   if (rc != NSD_OK || n_combine == 0) return rc;
   const int32_t* crec = plan_host + plan_host[kPlanOffCombines];
   bool packed = kUseCombineTable && n_combine <= kCombineTableMax;
+  int most_slots = 0;
+  for (int c = 0; c < n_combine; ++c) most_slots = std::max(most_slots, (int)crec[kPieceWords * c + kCombSlots]);
   CombineTable tab;
   for (int c = 0; packed && c < n_combine; ++c) {
     const int32_t* r = crec + kPieceWords * c;
@@ -975,10 +1082,17 @@ int paged_attention_impl(const void* q, void* o, float* lse, const void* k_cache
     tab.e[c] = (uint64_t)r[kCombFirst] | (uint64_t)r[kCombSlots] << 20 | (uint64_t)r[kCombHead] << 28 |
                (uint64_t)r[kCombRowStart] << 36 | (uint64_t)r[kCombQLen] << 56;
   }
-  if (packed)
-    hipLaunchKernelGGL(combine_table_kernel, dim3(n_combine, nt), dim3(256), 0, st, args, tab);
-  else
-    hipLaunchKernelGGL(combine_kernel, dim3(n_combine * nt), dim3(256), 0, st, args, nt);
+  auto merge = [&](auto slc) {
+    constexpr int SL = decltype(slc)::value;
+    const int groups = (rows_max * SL + 15) / 16;
+    if (packed)
+      hipLaunchKernelGGL(combine_table_kernel<SL>, dim3(n_combine, groups), dim3(256), 0, st, args, tab);
+    else
+      hipLaunchKernelGGL(combine_kernel<SL>, dim3(n_combine * groups), dim3(256), 0, st, args, groups);
+  };
+  if (most_slots <= kMergeSlots) merge(std::integral_constant<int, 1>{});
+  else if (most_slots <= 4 * kMergeSlots) merge(std::integral_constant<int, 4>{});
+  else merge(std::integral_constant<int, 16>{});
   return launch_status("paged_attention: partial merge");
 }
 
