@@ -79,6 +79,25 @@ __device__ inline f16x4 ds_read_tr16(const lds_char* p) {
   return __builtin_bit_cast(f16x4, t);
 }
 
+// Host: f(integral_constant<int, splits>), splits in 1 .. 8 (a projection's
+// split partials).  A kernel that knows the count at compile time has all the
+// splits' loads in flight at once; a loop over the count waits for each split
+// before the next one's load, a trip to memory per split in kernels that are
+// little more than one.
+template <typename F>
+inline void with_splits(int splits, F&& f) {
+  switch (splits) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
+  }
+}
+
 // Calls f(integral_constant<int, i>) for i = 0 .. N-1 (compile-time unrolled).
 template <int N, typename F, int... I>
 __device__ inline void static_for_impl(F&& f, std::integer_sequence<int, I...>) {

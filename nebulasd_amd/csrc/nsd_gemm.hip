@@ -401,16 +401,27 @@ __global__ __launch_bounds__(S::kThreads) void stream_gemm_kernel(const f16* __r
 }
 
 // y[i] = fp16(sum over splits of part[s][i]), eight elements per thread.
-__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, int splits,
-                                                           int64_t per_split, f16* __restrict__ y) {
+template <int S>
+__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ part, int64_t per_split,
+                                                           f16* __restrict__ y) {
   for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < per_split / 8; v += (int64_t)gridDim.x * 256) {
-    f32x4 lo = *reinterpret_cast<const f32x4*>(part + 8 * v);
-    f32x4 hi = *reinterpret_cast<const f32x4*>(part + 8 * v + 4);
-    for (int s = 1; s < splits; ++s) {
-      lo += *reinterpret_cast<const f32x4*>(part + s * per_split + 8 * v);
-      hi += *reinterpret_cast<const f32x4*>(part + s * per_split + 8 * v + 4);
+    f32x4 lo[S], hi[S];  // the splits' loads go out together
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      lo[s] = *reinterpret_cast<const f32x4*>(part + s * per_split + 8 * v);
+      hi[s] = *reinterpret_cast<const f32x4*>(part + s * per_split + 8 * v + 4);
     }
-    f16x8 h = {(f16)lo[0], (f16)lo[1], (f16)lo[2], (f16)lo[3], (f16)hi[0], (f16)hi[1], (f16)hi[2], (f16)hi[3]};
+#pragma unroll
+    for (int s = 1; s < S; ++s) {
+      lo[0] += lo[s];
+      hi[0] += hi[s];
+    }
+    f16x8 h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      h[e] = (f16)lo[0][e];
+      h[e + 4] = (f16)hi[0][e];
+    }
     *reinterpret_cast<f16x8*>(y + 8 * v) = h;
   }
 }
@@ -637,7 +648,9 @@ extern "C" int nsd_sum_partials(const float* partials, int splits, void* y, int6
     return fail(NSD_ERR_UNSUPPORTED, "sum_partials: pointers must be 16-byte aligned");
   const int64_t per = n_rows * n_out;
   const unsigned grid = (unsigned)std::min<int64_t>((per / 8 + 255) / 256, 1024);
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(grid), dim3(256), 0, as_stream(stream), partials, splits, per,
-                     static_cast<f16*>(y));
+  with_splits(splits, [&](auto count) {
+    hipLaunchKernelGGL(sum_partials_kernel<decltype(count)::value>, dim3(grid), dim3(256), 0, as_stream(stream),
+                       partials, per, static_cast<f16*>(y));
+  });
   return launch_status("sum_partials");
 }

@@ -34,41 +34,66 @@ typedef __attribute__((address_space(1))) u32x4 gbl_u32x4;
 __device__ inline f16x8 as_h8(u32x4 v) { return __builtin_bit_cast(f16x8, v); }
 __device__ inline u32x4 as_u4(f16x8 v) { return __builtin_bit_cast(u32x4, v); }
 
-// With `part` set, x is the projection whose fp32 split partials part holds
-// ([splits][rows][hidden]): summed in split order and rounded to fp16 (the
+// With SPLITS > 0, x is the projection whose fp32 split partials part holds
+// ([SPLITS][rows][hidden]): summed in split order and rounded to fp16 (the
 // GEMM's output rounding) in place of reading x; the normalised row is
-// written to x either way.
-template <int VPT>
+// written to x either way.  At decode batches the kernel is a trip to memory
+// and little else, so every load of the row goes out before the first use
+// (SPLITS known at compile time): over four splits, 4 x 1024 3.1 -> 2.6 us, 80 x
+// 4096 5.1 -> 4.8.
+template <int VPT, int SPLITS>
 __global__ void __launch_bounds__(kNormThreads)
 fused_add_rmsnorm_kernel(f16* __restrict__ x, f16* __restrict__ res, const f16* __restrict__ w, int nvec,
-                         int hidden, float eps, const float* __restrict__ part, int splits, int64_t split_stride) {
+                         int hidden, float eps, const float* __restrict__ part, int64_t split_stride) {
   __shared__ float s_part[kNormThreads / kWave];
   const int64_t row = blockIdx.x;
   u32x4* xr = reinterpret_cast<u32x4*>(x + row * hidden);
   u32x4* rr = reinterpret_cast<u32x4*>(res + row * hidden);
   const u32x4* wr = reinterpret_cast<const u32x4*>(w);
+  f16x8 a[VPT], b[VPT], wv[VPT];
+  f32x4 v[VPT][SPLITS > 0 ? SPLITS : 1][2];
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    const int i = threadIdx.x + j * kNormThreads;
+    if (i < nvec) {
+      if constexpr (SPLITS > 0) {
+        const float* p = part + row * hidden + 8 * i;
+#pragma unroll
+        for (int q = 0; q < SPLITS; ++q) {
+          v[j][q][0] = *reinterpret_cast<const f32x4*>(p + q * split_stride);
+          v[j][q][1] = *reinterpret_cast<const f32x4*>(p + q * split_stride + 4);
+        }
+      } else {
+        a[j] = as_h8(xr[i]);
+      }
+      b[j] = as_h8(rr[i]);
+      wv[j] = as_h8(wr[i]);
+    }
+  }
+  if constexpr (SPLITS > 0) {
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+#pragma unroll
+      for (int q = 1; q < SPLITS; ++q) {
+        v[j][0][0] += v[j][q][0];
+        v[j][0][1] += v[j][q][1];
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a[j][e] = (f16)v[j][0][0][e];
+        a[j][e + 4] = (f16)v[j][0][1][e];
+      }
+    }
+  }
   f16x8 s[VPT];
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * kNormThreads;
     if (i < nvec) {
-      f16x8 a;
-      if (part != nullptr) {
-        const float* p = part + row * hidden + 8 * i;
-        f32x4 lo = *reinterpret_cast<const f32x4*>(p), hi = *reinterpret_cast<const f32x4*>(p + 4);
-        for (int q = 1; q < splits; ++q) {
-          lo += *reinterpret_cast<const f32x4*>(p + q * split_stride);
-          hi += *reinterpret_cast<const f32x4*>(p + q * split_stride + 4);
-        }
-        a = f16x8{(f16)lo[0], (f16)lo[1], (f16)lo[2], (f16)lo[3], (f16)hi[0], (f16)hi[1], (f16)hi[2], (f16)hi[3]};
-      } else {
-        a = as_h8(xr[i]);
-      }
-      const f16x8 b = as_h8(rr[i]);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        s[j][e] = (f16)((float)a[e] + (float)b[e]);  // one fp16 rounding, as an fp16 add
+        s[j][e] = (f16)((float)a[j][e] + (float)b[j][e]);  // one fp16 rounding, as an fp16 add
         const float f = (float)s[j][e];
         ss += f * f;
       }
@@ -86,10 +111,9 @@ fused_add_rmsnorm_kernel(f16* __restrict__ x, f16* __restrict__ res, const f16* 
   for (int j = 0; j < VPT; ++j) {
     const int i = threadIdx.x + j * kNormThreads;
     if (i < nvec) {
-      const f16x8 wv = as_h8(wr[i]);
       f16x8 o;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = (f16)((float)s[j][e] * rstd * (float)wv[e]);
+      for (int e = 0; e < 8; ++e) o[e] = (f16)((float)s[j][e] * rstd * (float)wv[j][e]);
       xr[i] = as_u4(o);
     }
   }
@@ -655,17 +679,22 @@ static int fused_add_rmsnorm(void* x, void* residual, const void* weight, int64_
   if (n_rows > INT32_MAX) return fail(NSD_ERR_UNSUPPORTED, "fused_add_rmsnorm: too many rows");
   const int nvec = (int)(hidden / 8);
   const int vpt = (nvec + kNormThreads - 1) / kNormThreads;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)n_rows), dim3(kNormThreads), 0, as_stream(stream),
-                       static_cast<f16*>(x), static_cast<f16*>(residual), static_cast<const f16*>(weight), nvec,
-                       (int)hidden, eps, part, splits, n_rows * hidden);
+  auto go = [&](auto count) {
+    constexpr int S = decltype(count)::value;
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)n_rows), dim3(kNormThreads), 0, as_stream(stream), static_cast<f16*>(x),
+                         static_cast<f16*>(residual), static_cast<const f16*>(weight), nvec, (int)hidden, eps, part,
+                         n_rows * hidden);
+    };
+    switch (vpt) {
+      case 1: launch(fused_add_rmsnorm_kernel<1, S>); break;
+      case 2: launch(fused_add_rmsnorm_kernel<2, S>); break;
+      case 3: launch(fused_add_rmsnorm_kernel<3, S>); break;
+      default: launch(fused_add_rmsnorm_kernel<4, S>); break;
+    }
   };
-  switch (vpt) {
-    case 1: go(fused_add_rmsnorm_kernel<1>); break;
-    case 2: go(fused_add_rmsnorm_kernel<2>); break;
-    case 3: go(fused_add_rmsnorm_kernel<3>); break;
-    default: go(fused_add_rmsnorm_kernel<4>); break;
-  }
+  if (part == nullptr) go(std::integral_constant<int, 0>{});
+  else with_splits(splits, go);
   return launch_status("fused_add_rmsnorm");
 }
 

@@ -258,7 +258,10 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(u32x4* __restrict__ q, 
 // fp32 split partials [splits][rows][q_stride] (q_stride = (hq + 2 hkv) D):
 // each element is summed in split order and rounded to fp16 (the GEMM's
 // output rounding) where it would be read, and k is written to the cache
-// only.
+// only.  SPLITS: their number, 0 for fp16 rows; the splits' loads go out
+// together, before the row's slot is looked up (80 rows of 48 heads over five
+// splits 5.9 -> 4.9 us).
+template <int SPLITS>
 __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
     const f16* q, int64_t q_stride, f16* q_out, f16* k, int64_t k_stride, const f16* __restrict__ v,
     int64_t v_stride,
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
     f16* __restrict__ kc, f16* __restrict__ vc, const int32_t* __restrict__ bt, int64_t bt_rows,
     int64_t bt_stride, const int32_t* __restrict__ seq_ids, const int32_t* __restrict__ seq_lens,
     int64_t n_rows, int64_t num_blocks, int num_layers, int layer, int hq, int hkv,
-    int32_t* status, const float* __restrict__ part, int splits) {
+    int32_t* status, const float* __restrict__ part) {
   const int lane = threadIdx.x & 63;
   const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int heads = hq + 2 * hkv;
@@ -275,12 +278,21 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
   const int64_t r = wid / heads;
   const int hd = (int)(wid % heads);
   const int64_t pos = (int64_t)seq_lens[r] - 1;
-  // element c of head hd of this row from the partials, as the GEMM's fp16 output
-  const int64_t split_stride = n_rows * q_stride;
-  auto from_part = [&](int c) {
-    const float* p = part + r * q_stride + (int64_t)hd * D + c;
+  // elements lane and lane + 64 of head hd of this row from the partials, as
+  // the GEMM's fp16 output
+  float p0[SPLITS > 0 ? SPLITS : 1], p1[SPLITS > 0 ? SPLITS : 1];
+  if constexpr (SPLITS > 0) {
+    const float* p = part + r * q_stride + (int64_t)hd * D + lane;
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s) {
+      p0[s] = p[s * n_rows * q_stride];
+      p1[s] = p[s * n_rows * q_stride + 64];
+    }
+  }
+  auto from_part = [&](const float* p) {
     float acc = p[0];
-    for (int q2 = 1; q2 < splits; ++q2) acc += p[q2 * split_stride];
+#pragma unroll
+    for (int s = 1; s < SPLITS; ++s) acc += p[s];
     return f16_of(acc);
   };
 
@@ -301,10 +313,10 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
   if (hd >= hq + hkv) {  // v head: bit-exact copy of 256 bytes
     const int h = hd - hq - hkv;
     if (slot >= 0) {
-      if (part != nullptr) {
+      if constexpr (SPLITS > 0) {
         f16* dst = vc + slot + (int64_t)h * BS * D;
-        dst[lane] = from_part(lane);
-        dst[lane + 64] = from_part(lane + 64);
+        dst[lane] = from_part(p0);
+        dst[lane + 64] = from_part(p1);
       } else {
         const uint32_t* src = reinterpret_cast<const uint32_t*>(v + r * v_stride + (int64_t)h * D);
         uint32_t* dst = reinterpret_cast<uint32_t*>(vc + slot + (int64_t)h * BS * D);
@@ -319,12 +331,12 @@ __global__ __launch_bounds__(256) void qk_norm_rope_store_kernel(
   }
   const bool isk = hd >= hq;
   const int h = isk ? hd - hq : hd;
-  f16* x = isk ? (part != nullptr ? nullptr : k + r * k_stride + (int64_t)h * D) : q_out + (r * hq + h) * D;
+  f16* x = isk ? (SPLITS > 0 ? nullptr : k + r * k_stride + (int64_t)h * D) : q_out + (r * hq + h) * D;
   const f16* w = isk ? kw : qw;
   float x0, x1;
-  if (part != nullptr) {
-    x0 = (float)from_part(lane);
-    x1 = (float)from_part(lane + 64);
+  if constexpr (SPLITS > 0) {
+    x0 = (float)from_part(p0);
+    x1 = (float)from_part(p1);
   } else {
     const f16* xin = isk ? k + r * k_stride + (int64_t)h * D : q + r * q_stride + (int64_t)h * D;
     x0 = (float)xin[lane];
@@ -492,14 +504,18 @@ static int qk_norm_rope_store_impl(const void* q, int64_t q_stride, void* q_out,
       v_stride < (int64_t)num_kv_heads * D || (q_stride | k_stride | v_stride) & 1)
     return fail(NSD_ERR_INVALID, "qk_norm_rope_store: row strides must be even and cover the heads");
   const int64_t waves = n_rows * (num_q_heads + 2 * num_kv_heads);
-  hipLaunchKernelGGL(qk_norm_rope_store_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
-                     as_stream(stream), static_cast<const f16*>(q), q_stride, static_cast<f16*>(q_out),
-                     static_cast<f16*>(k), k_stride, static_cast<const f16*>(v), v_stride,
-                     static_cast<const f16*>(q_norm_w), static_cast<const f16*>(k_norm_w), eps,
-                     static_cast<const f16*>(cos_cache), static_cast<const f16*>(sin_cache), n_positions,
-                     static_cast<f16*>(k_cache), static_cast<f16*>(v_cache), block_table, bt_rows, bt_stride,
-                     seq_ids, seq_lens, n_rows, num_blocks, num_layers, layer, num_q_heads, num_kv_heads,
-                     status, part, splits);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,
+                       as_stream(stream), static_cast<const f16*>(q), q_stride, static_cast<f16*>(q_out),
+                       static_cast<f16*>(k), k_stride, static_cast<const f16*>(v), v_stride,
+                       static_cast<const f16*>(q_norm_w), static_cast<const f16*>(k_norm_w), eps,
+                       static_cast<const f16*>(cos_cache), static_cast<const f16*>(sin_cache), n_positions,
+                       static_cast<f16*>(k_cache), static_cast<f16*>(v_cache), block_table, bt_rows, bt_stride,
+                       seq_ids, seq_lens, n_rows, num_blocks, num_layers, layer, num_q_heads, num_kv_heads,
+                       status, part);
+  };
+  if (part == nullptr) launch(qk_norm_rope_store_kernel<0>);
+  else with_splits(splits, [&](auto count) { launch(qk_norm_rope_store_kernel<decltype(count)::value>); });
   return launch_status("qk_norm_rope_store");
 }
 
