@@ -440,17 +440,9 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
   const int lg = lane >> 4;   // k-group of the MFMA operands
   const int n_rows = q_len * a.gqa;
 
-  // Block ids of this wave's blocks (block wave + 4i on lane i); ids outside
-  // the pool read block 0 and are masked.
-  int64_t boff = 0;
-  bool bad = false;
-  if (lane < my_n) {
-    const int id = tabled ? tab_id : a.bt[(int64_t)rv[kPieceSeqId] * a.bt_stride + blk0 + wave + kWaves * lane];
-    bad = id < 0 || id >= a.num_blocks;
-    boff = (int64_t)(bad ? 0 : id) * a.blk_stride + ((int64_t)a.layer * a.hkv + head) * BS * D;
-  }
-  const uint64_t bad_mask = __builtin_amdgcn_ballot_w64(bad);
-  if (bad_mask != 0 && lane == 0) flag_status(a.status, NSD_STATUS_BAD_BLOCK);
+  // Block ids of this wave's blocks (block wave + 4i on lane i).
+  int blk_id = tab_id;
+  if (!tabled && lane < my_n) blk_id = a.bt[(int64_t)rv[kPieceSeqId] * a.bt_stride + blk0 + wave + kWaves * lane];
 
   // DMA sources: load c of a tile fills rows 4c .. 4c+3 (lane l: row 4c + l/16,
   // stored chunk l % 16), fetching the chunk the swizzle puts there.
@@ -461,36 +453,11 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
     ksrc[c] = t * D + (((lane & 15) ^ swz_k(t)) << 3);
     vsrc[c] = t * D + (((lane & 15) ^ swz_v(t)) << 3);
   }
-  auto issue = [&](int jj) __attribute__((always_inline)) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, jj);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), jj);
-    const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
-    const f16* kb = a.k_cache + off;
-    const f16* vb = a.v_cache + off;
-    const uint32_t slot = lds_base + (jj & 1) * kSlot;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's earlier reads are done
-#pragma unroll
-    for (int c = 0; c < 4; ++c) dma_load(slot + c * 1024, kb + ksrc[c]);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) dma_load(slot + kTile + c * 1024, vb + vsrc[c]);
-  };
-  // one half of block jj's slot: its K tile (v = false) or its V tile
-  auto issue_half = [&](int jj, bool v) __attribute__((always_inline)) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, jj);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), jj);
-    const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
-    const f16* b = (v ? a.v_cache : a.k_cache) + off;
-    const uint32_t dst = lds_base + (jj & 1) * kSlot + (v ? kTile : 0);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this half's earlier reads are done
-#pragma unroll
-    for (int c = 0; c < 4; ++c) dma_load(dst + c * 1024, b + (v ? vsrc[c] : ksrc[c]));
-  };
-
-  // The first two blocks' loads go out before the query rows', so the rows
-  // arrive under the blocks' latency; then everything issued so far has
-  // landed (the builtin also tells the compiler its own loads are done, so
-  // it inserts no wait for them inside the loop, which would drain the
-  // buffer loads too: vmcnt retires in order).
+  // Start, without the prologue: the first two blocks' loads go out before
+  // the query rows', so the rows arrive under the blocks' latency; then
+  // everything issued so far has landed (the builtin also tells the compiler
+  // its own loads are done, so it inserts no wait for them inside the loop,
+  // which would drain the buffer loads too: vmcnt retires in order).
   //
   // Fused prologue.  Rows are computed in the layout of the score MFMA's B
   // operand: lane (lg, lr) holds dims 32kk + 8lg .. +7 of its row (kk < 4),
@@ -502,11 +469,18 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
   //
   // New K/V rows: token i of the group sits at position ctx + i of its
   // sequence, in block (ctx + i) / 16.  The wave that streams such a block
-  // writes the block's new rows (lane row lr: token own_lo + lr) and has
-  // those stores done before it issues the block's DMA: before its first two
-  // blocks' loads when the block is one of those, else under the start's
-  // wait.  The tokens span at most four consecutive blocks, so a wave owns
-  // at most one of them.
+  // computes the block's new rows (lane row lr: token own_lo + lr) and stores
+  // them to the cache.  The tokens span at most four consecutive blocks, so a
+  // wave owns at most one of them.
+  //
+  // Order: the rows' loads go out beside the block ids', and once both are
+  // in the first two blocks' DMA; the norms and rotations then run under the
+  // DMA's latency.  When the wave's own block is one of those two, the DMA
+  // reads the new tokens' rows before they are stored, so the wave also
+  // writes them into its LDS slot once the block has landed: waiting for the
+  // stores before the DMA cost a trip to memory (4 requests of up to 256
+  // tokens: 11.6 -> 10.2 us a launch).  A later block's DMA follows the start's wait, which
+  // covers the stores.
   int own_jj = -1, own_lo = 0, own_hi = 0;
   if constexpr (FUSED) {
     const int b_first = ctx / BS, b_last = (ctx + q_len - 1) / BS;
@@ -519,40 +493,50 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
       }
     }
   }
-  // a bad block is flagged above and gets no stores
-  const bool own = FUSED && own_jj >= 0 && !((bad_mask >> own_jj) & 1);
   // One row of head hd (Hq q heads, then Hkv k, then Hkv v) of the q/k/v
   // projection's fp16 output, in the row layout.
   auto load_row = [&](int64_t r, int hd, f16x8 (&h)[4]) __attribute__((always_inline)) {
     if constexpr (FUSED) {
-      if (fx.part == nullptr) {
-        const f16* src = hd < a.hq ? fx.q + r * fx.q_rs + (int64_t)hd * D
-                         : hd < a.hq + a.hkv ? fx.k + r * fx.k_rs + (int64_t)(hd - a.hq) * D
-                                             : fx.v + r * fx.v_rs + (int64_t)(hd - a.hq - a.hkv) * D;
+      const f16* src = hd < a.hq ? fx.q + r * fx.q_rs + (int64_t)hd * D
+                       : hd < a.hq + a.hkv ? fx.k + r * fx.k_rs + (int64_t)(hd - a.hq) * D
+                                           : fx.v + r * fx.v_rs + (int64_t)(hd - a.hq - a.hkv) * D;
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) h[kk] = *reinterpret_cast<const f16x8*>(src + 32 * kk + 8 * lg);
-      } else {
-        // the splits summed in split order, a split's eight loads together
-        const float* prow = fx.part + r * fx.part_rs + (int64_t)hd * D + 8 * lg;
-        f32x4 acc[8];
+      for (int kk = 0; kk < 4; ++kk) h[kk] = *reinterpret_cast<const f16x8*>(src + 32 * kk + 8 * lg);
+    }
+  };
+  // The same row from the split partials, in two parts so that a caller has
+  // several rows' first two splits in flight; the splits are added in split
+  // order and rounded to fp16.
+  struct Splits {
+    f32x4 first[8], second[8];
+  };
+  auto load_split = [&](int64_t r, int hd, int s2, f32x4 (&v)[8]) __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      const float* ps = fx.part + r * fx.part_rs + (int64_t)hd * D + 8 * lg + (int64_t)s2 * fx.split_stride;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) acc[c] = *reinterpret_cast<const f32x4*>(prow + 32 * (c >> 1) + 4 * (c & 1));
-        for (int s2 = 1; s2 < fx.splits; ++s2) {
-          const float* ps = prow + (int64_t)s2 * fx.split_stride;
-          f32x4 add[8];
+      for (int c = 0; c < 8; ++c) v[c] = *reinterpret_cast<const f32x4*>(ps + 32 * (c >> 1) + 4 * (c & 1));
+    }
+  };
+  auto load_splits = [&](int64_t r, int hd, Splits& v) __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      load_split(r, hd, 0, v.first);
+      if (fx.splits > 1) load_split(r, hd, 1, v.second);
+    }
+  };
+  auto sum_splits = [&](int64_t r, int hd, Splits& v, f16x8 (&h)[4]) __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      for (int s2 = 1; s2 < fx.splits; ++s2) {
+        if (s2 > 1) load_split(r, hd, s2, v.second);
 #pragma unroll
-          for (int c = 0; c < 8; ++c) add[c] = *reinterpret_cast<const f32x4*>(ps + 32 * (c >> 1) + 4 * (c & 1));
-#pragma unroll
-          for (int c = 0; c < 8; ++c) acc[c] += add[c];
-        }
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            h[kk][j] = f16_of(acc[2 * kk][j]);
-            h[kk][j + 4] = f16_of(acc[2 * kk + 1][j]);
-          }
+        for (int c = 0; c < 8; ++c) v.first[c] += v.second[c];
       }
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          h[kk][j] = f16_of(v.first[2 * kk][j]);
+          h[kk][j + 4] = f16_of(v.first[2 * kk + 1][j]);
+        }
     }
   };
   // the norm weights of a row (any readable row when there is no norm)
@@ -608,38 +592,88 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
         out[kk + 2][j] = f16_of(rope_hi(x[kk][j], x[kk + 2][j], c, sn));
       }
   };
-  f16x8 nk[4], nv[4], nkw[4], ncs[4];  // the new rows' k, v, k-norm weights, angles
+  // the new rows' k (then normalised and rotated), v, k-norm weights, angles
+  f16x8 nk[4], nv[4], nkw[4], ncs[4];
   auto load_new = [&]() __attribute__((always_inline)) {
     if constexpr (FUSED) {
       const int i = own_lo + lr < own_hi ? own_lo + lr : own_lo;
-      load_row(row_start + i, a.hq + head, nk);
-      load_row(row_start + i, a.hq + a.hkv + head, nv);
+      const int64_t r = row_start + i;
       load_w(fx.kn, nkw);
       load_cs(ctx + i, ncs);
-    }
-  };
-  auto store_new = [&]() __attribute__((always_inline)) {
-    if constexpr (FUSED) {
-      f16x8 ko[4];
-      norm_rope(nk, fx.kn != nullptr, nkw, ncs, ko);
-      if (own_lo + lr < own_hi) {
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, own_jj);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), own_jj);
-        const int64_t at = (int64_t)(((uint64_t)hi << 32) | lo) + (int64_t)((ctx + own_lo + lr) % BS) * D;
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          *reinterpret_cast<f16x8*>(fx.kc + at + 32 * kk + 8 * lg) = ko[kk];
-          *reinterpret_cast<f16x8*>(fx.vc + at + 32 * kk + 8 * lg) = nv[kk];
-        }
+      if (fx.part == nullptr) {
+        load_row(r, a.hq + head, nk);
+        load_row(r, a.hq + a.hkv + head, nv);
+      } else {
+        Splits k, v;
+        load_splits(r, a.hq + head, k);
+        load_splits(r, a.hq + a.hkv + head, v);
+        sum_splits(r, a.hq + head, k, nk);
+        sum_splits(r, a.hq + a.hkv + head, v, nv);
       }
     }
   };
-  const bool own_early = own && own_jj <= 1;
-  if (own_early) {
-    load_new();
-    store_new();
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the new rows are in the cache before their block's DMA
+  // the query row of this lane in row tile t; rows past the group as row 0
+  f16x8 qh[4], qcs[4], qw[4];
+  auto load_q = [&](int t) __attribute__((always_inline)) {
+    if constexpr (FUSED) {
+      const int n = 16 * t + lr, nr = n < n_rows ? n : 0;
+      const int qi = nr / a.gqa, gh = nr - qi * a.gqa;
+      load_w(fx.qn, qw);
+      load_cs(ctx + qi, qcs);
+      if (fx.part == nullptr) {
+        load_row(row_start + qi, head * a.gqa + gh, qh);
+      } else {
+        Splits v;
+        load_splits(row_start + qi, head * a.gqa + gh, v);
+        sum_splits(row_start + qi, head * a.gqa + gh, v, qh);
+      }
+    }
+  };
+  const bool builds = FUSED && wave < (NT == 1 ? kWaves : NT);  // one tile: every wave builds it
+  if constexpr (FUSED) {
+    if (own_jj >= 0) load_new();
+    if (builds) load_q(NT == 1 ? 0 : wave);
   }
+
+  // ids outside the pool read block 0 and are masked
+  int64_t boff = 0;
+  bool bad = false;
+  if (lane < my_n) {
+    bad = blk_id < 0 || blk_id >= a.num_blocks;
+    boff = (int64_t)(bad ? 0 : blk_id) * a.blk_stride + ((int64_t)a.layer * a.hkv + head) * BS * D;
+  }
+  const uint64_t bad_mask = __builtin_amdgcn_ballot_w64(bad);
+  if (bad_mask != 0 && lane == 0) flag_status(a.status, NSD_STATUS_BAD_BLOCK);
+  // a bad block is flagged and gets no stores
+  const bool own = FUSED && own_jj >= 0 && !((bad_mask >> own_jj) & 1);
+  const bool own_early = own && own_jj <= 1;
+
+  auto issue = [&](int jj) __attribute__((always_inline)) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, jj);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), jj);
+    const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
+    const f16* kb = a.k_cache + off;
+    const f16* vb = a.v_cache + off;
+    const uint32_t slot = lds_base + (jj & 1) * kSlot;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slot's earlier reads are done
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dma_load(slot + c * 1024, kb + ksrc[c]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dma_load(slot + kTile + c * 1024, vb + vsrc[c]);
+  };
+  // one half of block jj's slot: its K tile (v = false) or its V tile
+  auto issue_half = [&](int jj, bool v) __attribute__((always_inline)) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, jj);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), jj);
+    const int64_t off = (int64_t)(((uint64_t)hi << 32) | lo);
+    const f16* b = (v ? a.v_cache : a.k_cache) + off;
+    const uint32_t dst = lds_base + (jj & 1) * kSlot + (v ? kTile : 0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this half's earlier reads are done
+#pragma unroll
+    for (int c = 0; c < 4; ++c) dma_load(dst + c * 1024, b + (v ? vsrc[c] : ksrc[c]));
+  };
+
+  if constexpr (FUSED) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the rows are in: nothing below waits on them
   if (my_n > 0) issue(0);
   if (my_n > 1) issue(1);
   // Query rows of each row tile as the B operand of the score MFMA (lane
@@ -656,56 +690,59 @@ void paged_attn_kernel(AttnArgs a, PieceTable pt, Extra fx) {
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk) qf[t][kk] = *reinterpret_cast<const f16x8*>(qrow + 32 * kk + 8 * lg);
     }
-  } else if constexpr (NT == 1) {
-    // One row tile: every wave builds it (rows past the group read its row
-    // 0 and are never stored), its loads before its arithmetic; no barrier.
-    const bool own_late = own && !own_early;
-    if (own_late) load_new();
-    const int nr = lr < n_rows ? lr : 0;
-    const int qi = nr / a.gqa, gh = nr - qi * a.gqa;
-    f16x8 qh[4], qcs[4], qw[4];
-    load_w(fx.qn, qw);
-    load_row(row_start + qi, head * a.gqa + gh, qh);
-    load_cs(ctx + qi, qcs);
-    if (own_late) store_new();
-    norm_rope(qh, fx.qn != nullptr, qw, qcs, qf[0]);
   } else {
-    // Wave t < NT builds row tile t (rows past the group are zero and never
-    // stored) into the LDS after the buffers; after a barrier every wave
-    // reads all the tiles.  The wave's loads (the new rows', its tile's) go
-    // out before its arithmetic.
-    const bool own_late = own && !own_early;
-    if (own_late) load_new();
-    const bool builds = wave < NT;  // uniform over the wave
-    const int n = 16 * wave + lr;
-    f16x8 qh[4], qcs[4], qw[4];
-    if (builds) {
-      load_w(fx.qn, qw);
-      const int nr = n < n_rows ? n : 0;
-      const int qi = nr / a.gqa, gh = nr - qi * a.gqa;
-      if (n < n_rows) {
-        load_row(row_start + qi, head * a.gqa + gh, qh);
-      } else {
+    if (own) {
+      f16x8 ko[4];
+      norm_rope(nk, fx.kn != nullptr, nkw, ncs, ko);
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) qh[kk] = f16x8{};
+      for (int kk = 0; kk < 4; ++kk) nk[kk] = ko[kk];
+      if (own_lo + lr < own_hi) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)boff, own_jj);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)boff >> 32), own_jj);
+        const int64_t at = (int64_t)(((uint64_t)hi << 32) | lo) + (int64_t)((ctx + own_lo + lr) % BS) * D;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          *reinterpret_cast<f16x8*>(fx.kc + at + 32 * kk + 8 * lg) = nk[kk];
+          *reinterpret_cast<f16x8*>(fx.vc + at + 32 * kk + 8 * lg) = nv[kk];
+        }
       }
-      load_cs(ctx + qi, qcs);
     }
-    if (own_late) store_new();
-    lds_char* qlds = lds_all + kLdsBytes;
-    if (builds) {
-      f16x8 qo[4];
-      norm_rope(qh, fx.qn != nullptr, qw, qcs, qo);
+    if constexpr (NT == 1) {
+      norm_rope(qh, fx.qn != nullptr, qw, qcs, qf[0]);
+    } else {
+      // wave t < NT builds row tile t into the LDS after the buffers, and
+      // after a barrier (on LDS alone: the DMA stays in flight) every wave
+      // reads all the tiles
+      lds_char* qlds = lds_all + kLdsBytes;
+      if (builds) {
+        f16x8 qo[4];
+        norm_rope(qh, fx.qn != nullptr, qw, qcs, qo);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) *(lds_f16x8*)(qlds + ((wave * 4 + kk) * kWave + lane) * 16) = qo[kk];
+        for (int kk = 0; kk < 4; ++kk) *(lds_f16x8*)(qlds + ((wave * 4 + kk) * kWave + lane) * 16) = qo[kk];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) qf[t][kk] = *(const lds_f16x8*)(qlds + ((t * 4 + kk) * kWave + lane) * 16);
     }
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) qf[t][kk] = *(const lds_f16x8*)(qlds + ((t * 4 + kk) * kWave + lane) * 16);
   }
-  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+  if (own_early) {
+    // the two blocks have landed (all but the eight stores after them): the
+    // new rows over the cache's old ones, at their swizzled chunks
+    wait_vm<8>();
+    if (own_lo + lr < own_hi) {
+      const int t = (ctx + own_lo + lr) % BS;
+      lds_char* row = lds_all + wave * kWaveLds + (own_jj & 1) * kSlot + t * kRowBytes;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        *(lds_f16x8*)(row + (((4 * kk + lg) ^ swz_k(t)) << 4)) = nk[kk];
+        *(lds_f16x8*)(row + kTile + (((4 * kk + lg) ^ swz_v(t)) << 4)) = nv[kk];
+      }
+    }
+  } else {
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+  }
 
   // LDS read addresses (bytes within a slot): the score operand of k-step kk
   // (row lr, chunk 4kk + lg) and the transposing V read of dim tile mt (row
