@@ -47,6 +47,9 @@ __device__ inline void flag_status(int32_t* status, int32_t bit) {
   if (status != nullptr) atomicOr(status, bit);
 }
 
+// Compute units of the current device.
+int device_cus(int* cus);
+
 // Launch-status helper for the C ABI.
 inline int launch_status(const char* what) {
   hipError_t err = hipGetLastError();

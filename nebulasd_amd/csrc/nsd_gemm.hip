@@ -456,27 +456,6 @@ LinearConfig choose_linear(int64_t n, int64_t k, int cus) {
   return best;
 }
 
-// Compute units of the current device (queried once per device: the
-// decoder stack asks for every projection it enqueues).
-int device_cus(int* cus) {
-  constexpr int kMaxDevices = 64;
-  static std::atomic<int> cached[kMaxDevices];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess && dev >= 0 && dev < kMaxDevices) {
-    const int c = cached[dev].load(std::memory_order_relaxed);
-    if (c > 0) {
-      *cus = c;
-      return NSD_OK;
-    }
-  }
-  if (e == hipSuccess) e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e != hipSuccess) return fail(NSD_ERR_HIP, "linear: %s", hipGetErrorString(e));
-  if (*cus < 1) return fail(NSD_ERR_HIP, "linear: device %d reports %d compute units", dev, *cus);
-  if (dev >= 0 && dev < kMaxDevices) cached[dev].store(*cus, std::memory_order_relaxed);
-  return NSD_OK;
-}
-
 int check_linear(int64_t n_rows, int64_t n_out, int64_t n_in, const char* who) {
   if (n_rows < 1 || n_rows > 16 * kMaxRowTiles)
     return fail(NSD_ERR_UNSUPPORTED, "%s: n_rows=%lld outside [1, %d]", who, (long long)n_rows, 16 * kMaxRowTiles);
@@ -580,6 +559,27 @@ int gated_pairs(int64_t inter, int cus) {
 }
 
 }  // namespace
+
+// Compute units of the current device (queried once per device: the
+// decoder stack asks for every projection it enqueues).
+int device_cus(int* cus) {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cached[kMaxDevices];
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess && dev >= 0 && dev < kMaxDevices) {
+    const int c = cached[dev].load(std::memory_order_relaxed);
+    if (c > 0) {
+      *cus = c;
+      return NSD_OK;
+    }
+  }
+  if (e == hipSuccess) e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e != hipSuccess) return fail(NSD_ERR_HIP, "linear: %s", hipGetErrorString(e));
+  if (*cus < 1) return fail(NSD_ERR_HIP, "linear: device %d reports %d compute units", dev, *cus);
+  if (dev >= 0 && dev < kMaxDevices) cached[dev].store(*cus, std::memory_order_relaxed);
+  return NSD_OK;
+}
 
 int up_gate_silu_gated(const void* x, const void* up_gate, void* y, int64_t n_rows, int64_t hidden, int64_t inter,
                        void* stream, bool* served) {

@@ -10,11 +10,11 @@
 // h / (Hq/Hkv) (the repeat_interleave of transformer_layer.py:20-23).
 //
 // Work unit: (prompt, kv head, block of P = rows/gqa positions).  The
-// workgroup's query rows (128: four waves of 32) are the gqa q-heads of its
-// P positions, packed as row n = position_offset * gqa + head_in_group, so
-// every K/V tile staged in LDS serves all the q-heads that read it.  Three
-// workgroups share a compute unit, so one's loads and barriers overlap the
-// others' MFMAs.
+// workgroup's query rows (128: four waves of 32, or 64 where that leaves the
+// device too few workgroups) are the gqa q-heads of its P positions, packed as
+// row n = position_offset * gqa + head_in_group, so every K/V tile staged in
+// LDS serves all the q-heads that read it.  Three or four workgroups share a
+// compute unit, so one's loads and barriers overlap the others' MFMAs.
 //
 //   S^T[token][row] = K[token][:] . Q[row][:]            A = K (LDS), B = Q^T (registers)
 //   O^T[dim][row]  += V^T[dim][token] . P^T[token][row]  A = V^T (LDS), B = P^T (registers)
@@ -50,11 +50,12 @@ constexpr float kLazyMax = 8.f;
 
 // Kernel shape: NTW 16-row tiles per wave, NW waves per workgroup, KT tokens
 // per K/V tile, PF tiles of global loads in flight, LAZY running-max raise.
-template <int NTW_, int NW_, int KT_, int PF_, bool LAZY_, int WPE_ = 1>
+template <int NTW_, int NW_, int KT_, int PF_, bool LAZY_, int WPE_, int AHEAD_>
 struct PrefillCfg {
   static constexpr int NTW = NTW_, NW = NW_, KT = KT_, PF = PF_;
   static constexpr bool LAZY = LAZY_;
   static constexpr int WPE = WPE_;  // minimum waves per SIMD the register budget must allow
+  static constexpr int AHEAD = AHEAD_;  // V operands read ahead of the PV MFMAs (0: as the compiler orders them)
   static constexpr int rows = NW * 16 * NTW;  // query rows (position x q-head) per workgroup
   static constexpr int threads = NW * kWave;
   static constexpr int loads = 2 * KT * (PD / 8) / threads;  // 16-byte K/V loads per thread per tile
@@ -64,14 +65,28 @@ struct PrefillCfg {
   static_assert(KT % 32 == 0 && (PF == 1 || PF == 2), "tile shape");
 };
 
-// The shape every launch uses: 32 rows per wave, four waves, 32-token
-// tiles, three workgroups per compute unit (168 VGPRs).  Measured against
-// 8-wave workgroups (one per CU), 64-token tiles, a second tile in flight,
-// 16- and 64-row waves and the software-pipelined loop, all slower; shapes
-// that spill registers were slowest, and so was a software-pipelined loop
-// (K one tile ahead of V, the next tile's score MFMAs issued beside the
-// softmax).
-using PrefillShape = PrefillCfg<2, 4, 32, 1, true, 3>;
+// Two shapes, four waves each.  Measured against them: 8-wave workgroups (one
+// per CU), 64-token tiles, a second tile in flight, 64-row waves and a
+// software-pipelined loop (next tile's score MFMAs and last tile's PV beside
+// the softmax), all slower; shapes that spill registers were slowest.
+//
+// Wide: 32 rows per wave, 128 per workgroup, three workgroups per compute unit
+// (168 VGPRs).  With the device full the matrix cores and the vector units
+// share out the time (47% and 54% of the SIMD cycles, at the clock that power
+// allows: 1.02 PFLOP/s on two 8k prompts, where the library's 8192^3 matrix
+// product reaches 1.15).
+using PrefillWide = PrefillCfg<2, 4, 32, 1, true, 3, 0>;
+// Narrow: 16 rows per wave, 64 per workgroup, four workgroups per compute
+// unit (122 VGPRs), a tile's LDS reads issued ahead of their MFMAs.  A tile
+// step is a chain (LDS reads, scores, softmax, PV, barrier) that the wide
+// shape hides with its three workgroups per unit; with fewer than that on the
+// device, a call lasts as long as its longest workgroup, and this one's step
+// is shorter: 0.6 against 1.05 us.  us, wide -> narrow, Qwen3-8B heads: one
+// prompt of 128 tokens 9.5 -> 6.6, 512 20.8 -> 13.7, 2000 64.8 -> 54.2; 4 x
+// 256 14.5 -> 11.4.  At 512 workgroups of the wide shape (two per unit) it is
+// even (16 x 128 tokens 15.0 -> 14.4, 2500 tokens 83 -> 75), at three per unit
+// it loses (3 x 1024 42.8 -> 44.1, 3500 tokens 125 -> 133).
+using PrefillNarrow = PrefillCfg<1, 4, 32, 1, true, 4, 4>;
 
 struct PrefillArgs {
   const f16* q;               // [T, Hq, D]
@@ -161,19 +176,36 @@ prefill_attn_kernel(PrefillArgs a) {
   asm volatile("" ::: "memory");
 
   // K/V tile staging through registers: thread chunk c -> (K or V, token,
-  // 16-byte part); tile u is loaded into stage[u % PF].
+  // 16-byte part); tile u is loaded into stage[u % PF].  A load is the tile's
+  // uniform base plus a 32-bit offset that stays the thread's; only the
+  // prompt's last tile, whose tokens past the prompt read its last row (they
+  // are masked), works its offsets out again.
   u32x4 stage[C::PF][LPT];
+  const uint32_t row_b = a.hkv * PD * 2;  // bytes between tokens
+  const uint32_t part_b = (threadIdx.x % (PD / 8)) * 16;
+  auto token_of = [&](int i) { return (int)((threadIdx.x + i * NTHR) / (PD / 8)) % KT; };
+  constexpr int LH = LPT / 2;  // K's loads, then V's: the same tokens
+  uint32_t off[LH];
+#pragma unroll
+  for (int i = 0; i < LH; ++i) off[i] = token_of(i) * row_b + part_b;
   auto load_tile = [&](auto sidx, int t) {
     constexpr int S = decltype(sidx)::value;
+    const int64_t at = ((int64_t)(start + t * KT) * a.hkv + kvh) * PD;
+    const char* kb = reinterpret_cast<const char*>(a.k + at);
+    const char* vb = reinterpret_cast<const char*>(a.v + at);
+    if ((t + 1) * KT <= len) {
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int c = threadIdx.x + i * NTHR;
-      const int kv = (i * NTHR) / (KT * (PD / 8));
-      const int tok = (c / (PD / 8)) % KT, part = c % (PD / 8);
-      const int tk = min(t * KT + tok, len - 1);  // past the prompt: masked, reads its last row
-      const f16* base = kv ? a.v : a.k;
-      stage[S][i] = *reinterpret_cast<const u32x4*>(base + ((int64_t)(start + tk) * a.hkv + kvh) * PD +
-                                                    part * 8);
+      for (int i = 0; i < LH; ++i) {
+        stage[S][i] = *reinterpret_cast<const u32x4*>(kb + off[i]);
+        stage[S][i + LH] = *reinterpret_cast<const u32x4*>(vb + off[i]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < LH; ++i) {
+        const uint32_t o = min(token_of(i), len - 1 - t * KT) * row_b + part_b;
+        stage[S][i] = *reinterpret_cast<const u32x4*>(kb + o);
+        stage[S][i + LH] = *reinterpret_cast<const u32x4*>(vb + o);
+      }
     }
   };
   auto store_tile = [&](auto sidx, int buf) {
@@ -188,12 +220,13 @@ prefill_attn_kernel(PrefillArgs a) {
   };
 
   float m[NTW], l[NTW];  // running max (scaled log2 domain); this lane's share of the sum
+  float neg_m[NTW];      // what the exponents add: -m, 0 while m is -inf
   f32x4 acc[NTW][8];     // O^T: dims 16dt + 4lg .. +3 of row 16j + lr
 #pragma unroll
   for (int j = 0; j < NTW; ++j) {
     m[j] = -INFINITY;
     l[j] = 0.f;
-
+    neg_m[j] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) acc[j][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -211,14 +244,38 @@ prefill_attn_kernel(PrefillArgs a) {
     for (int h = 0; h < KH; ++h)
 #pragma unroll
       for (int j = 0; j < NTW; ++j) s[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f16x8 kf[KH][4];
+    auto load_k = [&](int h, int kk) {
+      kf[h][kk] = *(const lds_f16x8*)(kb + (16 * h + lr) * PROWB + 64 * kk + 16 * lg);
+    };
+    if constexpr (C::AHEAD > 0) {
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int h = 0; h < KH; ++h) load_k(h, kk);
+      __builtin_amdgcn_sched_barrier(0);  // every K read before the first MFMA
+    }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
 #pragma unroll
       for (int h = 0; h < KH; ++h) {
-        const f16x8 kf = *(const lds_f16x8*)(kb + (16 * h + lr) * PROWB + 64 * kk + 16 * lg);
+        if constexpr (C::AHEAD == 0) load_k(h, kk);
 #pragma unroll
-        for (int j = 0; j < NTW; ++j) s[h][j] = mfma_k32(kf, qf[j][kk], s[h][j]);
+        for (int j = 0; j < NTW; ++j) s[h][j] = mfma_k32(kf[h][kk], qf[j][kk], s[h][j]);
       }
+    }
+    // V^T operand of dims 16 (i % 8) .. +15 and the i / 8-th 32 tokens
+    constexpr int NV = 8 * (KT / 32);
+    auto load_v = [&](int i) {
+      const lds_char* vsrc = vb + (32 * (i / 8) + 4 * lg + (lr >> 2)) * PROWB + 8 * (lr & 3) + 32 * (i % 8);
+      const f16x4 lo = ds_read_tr16(vsrc), hi = ds_read_tr16(vsrc + 16 * PROWB);
+      return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    f16x8 vf[C::AHEAD > 0 ? C::AHEAD : 1];
+    if constexpr (C::AHEAD > 0) {
+#pragma unroll
+      for (int i = 0; i < C::AHEAD; ++i) vf[i] = load_v(i);
+      __builtin_amdgcn_sched_barrier(0);  // the first V reads under the softmax
     }
     // Causal mask where the tile reaches the block's positions (it also
     // hides tokens past the prompt: they lie past every valid row).
@@ -258,6 +315,7 @@ prefill_attn_kernel(PrefillArgs a) {
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) acc[j][dt] *= alpha;
         m[j] = m_new;
+        neg_m[j] = m_new == -INFINITY ? 0.f : -m_new;
       }
     }
     // P^T in the PV operand layout: k-step ks holds tokens 32ks + 4lg + i and
@@ -265,30 +323,27 @@ prefill_attn_kernel(PrefillArgs a) {
     f16x8 pf[KT / 32][NTW];
 #pragma unroll
     for (int j = 0; j < NTW; ++j) {
-      const float m_use = m[j] == -INFINITY ? 0.f : m[j];
       float ps = 0.f;
 #pragma unroll
       for (int h = 0; h < KH; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(s[h][j][i], c, -m_use));
+          const float p = __builtin_amdgcn_exp2f(fmaf(s[h][j][i], c, neg_m[j]));
           ps += p;
           pf[h / 2][j][4 * (h % 2) + i] = (f16)p;
         }
       l[j] += ps;
     }
     // O^T += V^T . P^T, 16 dims and 32 tokens per MFMA.
+    if constexpr (C::AHEAD > 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int ks = 0; ks < KT / 32; ++ks) {
-      const lds_char* vsrc = vb + (32 * ks + 4 * lg + (lr >> 2)) * PROWB + 8 * (lr & 3);
+    for (int i = 0; i < NV; ++i) {
+      const f16x8 v = C::AHEAD > 0 ? vf[C::AHEAD > 0 ? i % C::AHEAD : 0] : load_v(i);
+      if constexpr (C::AHEAD > 0)
+        if (i + C::AHEAD < NV) vf[i % C::AHEAD] = load_v(i + C::AHEAD);
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) {
-        const f16x4 lo = ds_read_tr16(vsrc + 32 * dt);
-        const f16x4 hi = ds_read_tr16(vsrc + 16 * PROWB + 32 * dt);
-        const f16x8 vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-#pragma unroll
-        for (int j = 0; j < NTW; ++j) acc[j][dt] = mfma_k32(vf, pf[ks][j], acc[j][dt]);
-      }
+      for (int j = 0; j < NTW; ++j) acc[j][i % 8] = mfma_k32(v, pf[i / 8][j], acc[j][i % 8]);
+      if (C::AHEAD > 0 && i + C::AHEAD < NV) __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -375,9 +430,9 @@ extern "C" int nsd_prefill_attention(const void* q, const void* k, const void* v
     return fail(NSD_ERR_INVALID, "prefill_attention: num_q_heads=%d not a multiple of num_kv_heads=%d",
                 num_q_heads, num_kv_heads);
   const int gqa = num_q_heads / num_kv_heads;
-  if (PrefillShape::rows % gqa != 0)
+  if (PrefillWide::rows % gqa != 0)
     return fail(NSD_ERR_UNSUPPORTED, "prefill_attention: q-heads per kv head %d must divide %d", gqa,
-                PrefillShape::rows);
+                PrefillWide::rows);
   if (n_seqs < 0 || max_seqlen < 0 || total_tokens < 0)
     return fail(NSD_ERR_INVALID, "prefill_attention: negative size");
   if (n_seqs == 0 || max_seqlen == 0 || total_tokens == 0) return NSD_OK;
@@ -401,5 +456,12 @@ extern "C" int nsd_prefill_attention(const void* q, const void* k, const void* v
   args.gqa = gqa;
   args.max_seqlen = max_seqlen;
   args.scale_log2 = softmax_scale * 1.4426950408889634f;
-  return launch_prefill<PrefillShape>(args, as_stream(stream));
+  // Workgroups of the wide shape that have work (the last block of a prompt
+  // half full on average): up to nine for four compute units, the narrow one.
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  const int64_t wide = (total_tokens * gqa / PrefillWide::rows + n_seqs / 2) * num_kv_heads;
+  if (PrefillNarrow::rows % gqa == 0 && 4 * wide <= 9 * (int64_t)cus)
+    return launch_prefill<PrefillNarrow>(args, as_stream(stream));
+  return launch_prefill<PrefillWide>(args, as_stream(stream));
 }

@@ -64,6 +64,17 @@ def test_prefill_gqa_ratios(gpu, hq, hkv):
     check(w, o, lse, f"gqa {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("hq,hkv,fill", [(8, 8, 12), (16, 8, 12), (32, 8, 12), (64, 8, 0), (128, 1, 0)])
+def test_prefill_wide_shape_edges(gpu, hq, hkv, fill):
+    """The tile and position-block edges in the 128-row kernel shape: enough prompts beside them to fill the
+    device, or (128 q-heads on one kv head) a head group that only that shape takes."""
+    model = dict(QWEN3_8B, num_attention_heads=hq, num_key_value_heads=hkv)
+    lens = EDGE_LENS + [511] * fill
+    w = make_prefill_workload("prefill_target", 8, device=gpu, lens=lens, model=model)
+    o, lse = run_prefill(w)
+    check(w, o, lse, f"wide {hq}/{hkv}")
+
+
 def test_prefill_matches_torch_sdpa_loop(gpu):
     """The reference's own formulation on the same GPU (transformer_layer.py:7-32):
     per-prompt scaled_dot_product_attention(is_causal=True) after
