@@ -307,8 +307,9 @@ int nsd_paged_attention_noalloc(const void* q, void* o, float* lse, const void* 
  * is not (fully) computed.  Hq/Hkv must divide 128.
  * seq_order (optional, device int32 [n_seqs]): the prompts longest first (a
  * permutation of 0..n_seqs-1; any order is correct, this one balances the
- * shader engines); NULL visits them in order.  An entry outside
- * [0, n_seqs) sets NSD_STATUS_BAD_SEQ.
+ * shader engines).  An entry outside [0, n_seqs) sets NSD_STATUS_BAD_SEQ.
+ * NULL: up to 64 prompts the kernel orders the work itself (no better order
+ * can be given); more are visited as they come.
  */
 int nsd_prefill_attention(const void* q, const void* k, const void* v, void* o, float* lse,
                           const int32_t* cu_seqlens, const int32_t* seq_order, int n_seqs,

@@ -30,11 +30,13 @@
 // loads are issued before the previous tile's MFMAs and written to the other
 // buffer after them, one barrier per tile.  A row's running max is raised
 // lazily (only past a margin, after a wave-wide vote), so most tiles need no
-// cross-lane reduction and no rescaling of the accumulators.  Workgroups are issued from the
-// last position block down, so the longest ones (the most tiles under the
-// causal mask) start first; the q-blocks of one (prompt, kv head) are
-// n_seqs*Hkv workgroups apart, which keeps them on one XCD when that count
-// is a multiple of 8.
+// cross-lane reduction and no rescaling of the accumulators.  Workgroups are
+// issued from the last position block down, so the longest ones (the most
+// tiles under the causal mask) start first; a block's kv heads are consecutive
+// workgroups, which keeps a head on one XCD when their count is a multiple of
+// 8.
+#include <algorithm>
+
 #include "nsd_device.h"
 
 namespace nsd {
@@ -102,8 +104,25 @@ struct PrefillArgs {
   int positions;              // P = rows per workgroup / gqa
   int max_seqlen;
   int q_blocks;               // ceil(max_seqlen / P)
+  int compact;                // 1: workgroups for the non-empty position blocks only
   float scale_log2;           // softmax_scale * log2(e)
 };
+
+// Sum over the wave's 64 lanes, in every lane.
+template <int CTRL>
+__device__ inline int dpp_iadd(int v) {
+  return v + __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
+}
+__device__ inline int wave_isum(int v) {
+  v = dpp_iadd<0xB1>(v);   // quad_perm [1,0,3,2]
+  v = dpp_iadd<0x4E>(v);   // quad_perm [2,3,0,1]
+  v = dpp_iadd<0x141>(v);  // row_half_mirror
+  v = dpp_iadd<0x140>(v);  // row_mirror
+  const auto a = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = (int)a[0] + (int)a[1];
+  const auto b = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  return (int)b[0] + (int)b[1];
+}
 
 template <class C>
 __global__ void __launch_bounds__(C::threads) __attribute__((amdgpu_waves_per_eu(C::WPE)))
@@ -118,36 +137,74 @@ prefill_attn_kernel(PrefillArgs a) {
   const int lr = lane & 15;  // row of a 16-row tile (B/C column)
   const int lg = lane >> 4;  // k-group of the MFMA operands
 
-  // Work item, last position block first.
-  const int per_qb = a.n_seqs * a.hkv;
-  const int qb = a.q_blocks - 1 - (int)blockIdx.x / per_qb;
-  const int item = (int)blockIdx.x % per_qb;
-  const int pos = item / a.hkv, kvh = item - pos * a.hkv;
-  // With prompts longest first, a block level's non-empty items are
-  // consecutive (cyclically), so in-order dispatch spreads them over the
-  // shader engines; rotating each level by its index moves the longest
-  // prompts to another engine at every level instead of stacking one
-  // engine's slots with them.
-  const int rank = (pos + qb) % a.n_seqs;
-  const int seq = a.seq_order != nullptr ? a.seq_order[rank] : rank;
-  if (seq < 0 || seq >= a.n_seqs) {
-    if (threadIdx.x == 0) flag_status(a.status, NSD_STATUS_BAD_SEQ);
-    return;
-  }
-  const int start = a.cu_seqlens[seq];
-  const int end = a.cu_seqlens[seq + 1];
   const int P = a.positions;
-  const int p0 = qb * P;
-  if (start < 0 || end < start || start > a.total_tokens) {
-    if (qb == 0 && kvh == 0 && threadIdx.x == 0) flag_status(a.status, NSD_STATUS_BAD_SEQ);
-    return;
+  int seq, qb, kvh, start, len;
+  if (a.compact) {
+    // Work item i of the non-empty position blocks, the last (longest) blocks
+    // of all prompts first: level L holds block L of every prompt that has
+    // one, and sum over prompts max(blocks - 1 - L, 0) items come before it.
+    // Each wave holds one prompt per lane, finds the level by bisection and
+    // the prompt as the level's k-th.
+    const int i = (int)blockIdx.x / a.hkv;
+    kvh = (int)blockIdx.x - i * a.hkv;
+    int s0 = 0, n = 0;
+    bool bad = false;
+    if (lane < a.n_seqs) {
+      s0 = a.cu_seqlens[lane];
+      const int s1 = a.cu_seqlens[lane + 1];
+      bad = s0 < 0 || s1 < s0 || s0 > a.total_tokens;
+      // an end past the tokens is cut there (below)
+      n = bad ? 0 : (int)((int64_t)s1 < a.total_tokens ? s1 : a.total_tokens) - s0;
+      bad |= n > a.max_seqlen;  // positions past the longest prompt's blocks are not computed
+    }
+    if (blockIdx.x == 0 && wave == 0 && __any(bad) && lane == 0) flag_status(a.status, NSD_STATUS_BAD_SEQ);
+    const int blocks = min((n + P - 1) / P, a.q_blocks);
+    if (i >= wave_isum(blocks)) return;
+    int lo = 0, hi = a.q_blocks - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (__builtin_amdgcn_readfirstlane(wave_isum(max(blocks - 1 - mid, 0))) <= i) hi = mid;
+      else lo = mid + 1;
+    }
+    qb = lo;
+    const int k = i - __builtin_amdgcn_readfirstlane(wave_isum(max(blocks - 1 - qb, 0)));
+    const uint64_t level = __builtin_amdgcn_ballot_w64(blocks > qb);
+    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(level >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)level, 0));
+    seq = __builtin_ctzll(__builtin_amdgcn_ballot_w64(blocks > qb && below == k));
+    start = __builtin_amdgcn_readlane(s0, seq);
+    len = __builtin_amdgcn_readlane(n, seq);
+  } else {
+    // Work item, last position block first.
+    const int per_qb = a.n_seqs * a.hkv;
+    qb = a.q_blocks - 1 - (int)blockIdx.x / per_qb;
+    const int item = (int)blockIdx.x % per_qb;
+    const int pos = item / a.hkv;
+    kvh = item - pos * a.hkv;
+    // With prompts longest first, a block level's non-empty items are
+    // consecutive (cyclically), so in-order dispatch spreads them over the
+    // shader engines; rotating each level by its index moves the longest
+    // prompts to another engine at every level instead of stacking one
+    // engine's slots with them.
+    const int rank = (pos + qb) % a.n_seqs;
+    seq = a.seq_order != nullptr ? a.seq_order[rank] : rank;
+    if (seq < 0 || seq >= a.n_seqs) {
+      if (threadIdx.x == 0) flag_status(a.status, NSD_STATUS_BAD_SEQ);
+      return;
+    }
+    start = a.cu_seqlens[seq];
+    const int end = a.cu_seqlens[seq + 1];
+    if (start < 0 || end < start || start > a.total_tokens) {
+      if (qb == 0 && kvh == 0 && threadIdx.x == 0) flag_status(a.status, NSD_STATUS_BAD_SEQ);
+      return;
+    }
+    // An end past the tokens is cut there, as the reference's slices of
+    // q[:num_prefill_tokens] cut the last prompt (its cu_seqlens ends at the
+    // forward's token count, model.py:412-415).
+    len = (int)((int64_t)end < a.total_tokens ? end : a.total_tokens) - start;
+    if (qb == 0 && kvh == 0 && threadIdx.x == 0 && len > a.max_seqlen)
+      flag_status(a.status, NSD_STATUS_BAD_SEQ);  // positions past the grid's blocks are not computed
   }
-  // An end past the tokens is cut there, as the reference's slices of
-  // q[:num_prefill_tokens] cut the last prompt (its cu_seqlens ends at the
-  // forward's token count, model.py:412-415).
-  const int len = (int)((int64_t)end < a.total_tokens ? end : a.total_tokens) - start;
-  if (qb == 0 && kvh == 0 && threadIdx.x == 0 && len > a.max_seqlen)
-    flag_status(a.status, NSD_STATUS_BAD_SEQ);  // positions past the grid's blocks are not computed
+  const int p0 = qb * P;
   if (p0 >= len) return;
 
   const int p_end = min(p0 + P, len);      // one past the block's last valid position
@@ -409,7 +466,15 @@ int launch_prefill(PrefillArgs args, hipStream_t stream) {
   if (attr != hipSuccess) return fail(NSD_ERR_HIP, "prefill_attention: LDS attribute: %s", hipGetErrorString(attr));
   args.positions = C::rows / args.gqa;
   args.q_blocks = (args.max_seqlen + args.positions - 1) / args.positions;
-  const int64_t grid = (int64_t)args.q_blocks * args.n_seqs * args.hkv;
+  // Without a prompt order and with a lane for every prompt, the workgroups
+  // find the non-empty blocks themselves (at most one part block a prompt);
+  // else every (block level, prompt) pair has one, and those past their
+  // prompt's end exit: 1746 of 4096 for 16 prompts of U[128, 1024], which
+  // held the slots of the first levels.
+  args.compact = args.seq_order == nullptr && args.n_seqs <= kWave;
+  int64_t items = (int64_t)args.q_blocks * args.n_seqs;
+  if (args.compact) items = std::min<int64_t>(items, args.total_tokens / args.positions + args.n_seqs);
+  const int64_t grid = items * args.hkv;
   if (grid > INT32_MAX) return fail(NSD_ERR_UNSUPPORTED, "prefill_attention: grid of %lld workgroups", (long long)grid);
   hipLaunchKernelGGL(prefill_attn_kernel<C>, dim3((unsigned)grid), dim3(C::threads), C::lds_bytes, stream, args);
   return launch_status("prefill_attention");

@@ -17,6 +17,10 @@ from .. import _lib
 from ._util import StatusWord, ptr, require, require_cuda, stream_of
 
 
+# prompts up to which the kernel orders the work itself, a lane for each
+_LANES = 64
+
+
 def _longest_first(cu_seqlens: torch.Tensor) -> torch.Tensor:
     """Prompt indices, longest first (device int32, computed on the device with
     no host synchronisation).  Kept on the ``cu_seqlens`` tensor object itself
@@ -50,9 +54,10 @@ def _launch(q, k, v, o, cu_seqlens, max_seqlen: int, softmax_scale: float,
         if lse.numel() != tokens * hq:
             raise ValueError("lse must be [tokens, Hq]")
     status = StatusWord(q.device) if validate else None
-    order = _longest_first(cu_seqlens)
+    n_seqs = cu_seqlens.numel() - 1
+    order = None if n_seqs <= _LANES else _longest_first(cu_seqlens)
     _lib.call("nsd_prefill_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-              ptr(lse), cu_seqlens.data_ptr(), order.data_ptr(), cu_seqlens.numel() - 1,
+              ptr(lse), cu_seqlens.data_ptr(), ptr(order), n_seqs,
               int(max_seqlen), tokens,
               hq, hkv, d, float(softmax_scale), ptr(status.t) if status else None, stream_of(q))
     if status is not None:

@@ -75,6 +75,34 @@ def test_prefill_wide_shape_edges(gpu, hq, hkv, fill):
     check(w, o, lse, f"wide {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65])
+@pytest.mark.parametrize("long", [0, 900], ids=["narrow", "wide"])
+def test_prefill_prompt_counts(gpu, n, long):
+    """Prompts up to a lane each (64) and one more; empty prompts among them, a first prompt that does not start
+    at token 0, and a last one that the tokens cut short: rows of no prompt stay as they were."""
+    rng = np.random.default_rng(n)
+    lens = [int(x) for x in rng.integers(0, 70, n)]
+    lens[n // 2] += long if n < 8 else 0
+    lens[n - 1] += 40
+    if long and n >= 8:
+        lens = [x + 120 for x in lens]
+    lens[0] = 0 if n > 1 else lens[0]
+    skip, cut = 5, 9
+    w = make_prefill_workload("prefill_target", n, device=gpu, lens=[skip] + lens)
+    cu = (w.cu_seqlens[1:]).contiguous()
+    t = w.tokens - cut
+    o = torch.full((t,) + w.q.shape[1:], 7.0, dtype=torch.float16, device=gpu)
+    lse = torch.full(w.q.shape[:2], 7.0, dtype=torch.float32, device=gpu)[:t].contiguous()
+    from nebulasd_amd.kernels.prefill_attn import _launch
+    _launch(w.q[:t], w.k[:t], w.v[:t], o, cu, max(lens), 128 ** -0.5, lse, True)
+    torch.cuda.synchronize()
+    end = np.minimum(cu.cpu().numpy(), t)
+    wo, wl = oracle.prefill_attention(w.q[:t].cpu().numpy(), w.k[:t].cpu().numpy(), w.v[:t].cpu().numpy(), end)
+    assert_close(o[skip:].float().cpu().numpy(), wo[skip:], ATOL_O, RTOL_O, f"{n} prompts o")
+    assert_close(lse[skip:].cpu().numpy(), wl[skip:], ATOL_LSE, 0.0, f"{n} prompts lse")
+    assert (o[:skip] == 7).all() and (lse[:skip] == 7).all()
+
+
 def test_prefill_matches_torch_sdpa_loop(gpu):
     """The reference's own formulation on the same GPU (transformer_layer.py:7-32):
     per-prompt scaled_dot_product_attention(is_causal=True) after
