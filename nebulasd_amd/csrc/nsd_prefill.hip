@@ -42,8 +42,11 @@
 namespace nsd {
 namespace {
 
+typedef __attribute__((address_space(3))) f16x4 lds_f16x4;
+
 constexpr int PD = kHeadDim;        // 128
 constexpr int PROWB = PD * 2 + 32;  // LDS bytes per staged token row (32 B bank shift: no conflicts)
+constexpr int OROWB = PD * 2 + 16;  // LDS bytes per output row (16 B bank shift)
 constexpr float kLn2f = 0.69314718055994531f;
 // A row's running max is raised only when a tile's scores exceed it by more
 // than this (log2 units): the softmax terms then stay below 2^8, exact after
@@ -64,6 +67,7 @@ struct PrefillCfg {
   static constexpr int lds_bytes = 2 * 2 * KT * PROWB;       // [buffer][K, V][token][padded row]
   static_assert(loads * threads == 2 * KT * (PD / 8), "tile loads split evenly");
   static_assert((KT * (PD / 8)) % threads == 0, "each load is all-K or all-V");
+  static_assert(rows * (PD * 2 + 16) <= lds_bytes, "the output rows fit the tiles' LDS");
   static_assert(KT % 32 == 0 && (PF == 1 || PF == 2), "tile shape");
 };
 
@@ -432,27 +436,36 @@ prefill_attn_kernel(PrefillArgs a) {
     if (t + 1 < n_tiles) iteration(integral_constant<int, 1>{}, t + 1);
   }
 
-  // Normalise and write the valid rows.
+  // Normalise and write the valid rows, through the tiles' LDS (the last
+  // barrier is past its last read; each wave its own part) so that a store
+  // instruction writes whole 256-byte rows, the gqa heads of a position one
+  // after another, instead of 32-byte pieces of 16 rows: 16 prompts of U[128,
+  // 1024] 92 -> 88 us, 64 of 128 tokens 48 -> 42.  (The query rows brought in
+  // the same way made every call 1-4% slower.)
+  lds_char* mine = s_kv + wave * (16 * NTW * OROWB);
 #pragma unroll
   for (int j = 0; j < NTW; ++j) {
     float lt = l[j];
     lt += __shfl_xor(lt, 16, kWave);
     lt += __shfl_xor(lt, 32, kWave);
-    const int n = row0 + 16 * j + lr;
-    const int pq = n / a.gqa;
-    const int pos = p0 + pq;
-    if (pos >= len) continue;
-    const int head = kvh * a.gqa + (n - pq * a.gqa);
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
-    f16* op = a.o + ((int64_t)(start + pos) * a.hq + head) * PD + 4 * lg;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
       const f32x4 ov = acc[j][dt] * inv;
       const f16x4 hv = {(f16)ov[0], (f16)ov[1], (f16)ov[2], (f16)ov[3]};
-      *reinterpret_cast<f16x4*>(op + 16 * dt) = hv;
+      *(lds_f16x4*)(mine + (16 * j + lr) * OROWB + 32 * dt + 8 * lg) = hv;
     }
-    if (lg == 0 && a.lse != nullptr)
-      a.lse[(int64_t)(start + pos) * a.hq + head] = lt > 0.f ? (m[j] + __log2f(lt)) * kLn2f : -INFINITY;
+    const int n = row0 + 16 * j + lr, pq = n / a.gqa;
+    if (lg == 0 && a.lse != nullptr && p0 + pq < len)
+      a.lse[(int64_t)(start + p0 + pq) * a.hq + kvh * a.gqa + (n - pq * a.gqa)] =
+          lt > 0.f ? (m[j] + __log2f(lt)) * kLn2f : -INFINITY;
+  }
+#pragma unroll
+  for (int u = 0; u < 4 * NTW; ++u) {
+    const int r = 4 * u + (lane >> 4), n = row0 + r, pq = n / a.gqa;
+    if (p0 + pq < len)
+      *reinterpret_cast<u32x4*>(a.o + ((int64_t)(start + p0 + pq) * a.hq + kvh * a.gqa + (n - pq * a.gqa)) * PD +
+                                8 * (lane & 15)) = *(const lds_u32x4*)(mine + r * OROWB + 16 * (lane & 15));
   }
 }
 
