@@ -265,6 +265,7 @@ __device__ inline void merge_row_wide(const AttnArgs& a, int head, int first, in
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const float wgt = exp2f(ls[u] - use);
+      if (s0 + SL * u >= n_slots) h[u] = f16x8{};  // a repeated slot may hold an infinity: 0 * inf
       st.lo += f32x4{(float)h[u][0], (float)h[u][1], (float)h[u][2], (float)h[u][3]} * wgt;
       st.hi += f32x4{(float)h[u][4], (float)h[u][5], (float)h[u][6], (float)h[u][7]} * wgt;
       st.W += wgt;

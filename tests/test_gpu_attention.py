@@ -128,6 +128,19 @@ def test_attention_merge_of_many_pieces(gpu, model, q_len, ctxs):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
 
 
+@pytest.mark.parametrize("ctx", [1160, 4300, 9000], ids=["9 slots", "34", "64"])
+def test_attention_merge_keeps_an_infinity(gpu, ctx):
+    """An infinite value of the first token makes that dim of every row of its heads infinite, and nothing
+    else: no thread of the merge multiplies it by the zero weight of a slot that is not there."""
+    w = make_workload("target_verify", 9, device=gpu, pool_blocks=1200, num_layers=2, ctxs=[ctx], q_len=1,
+                      model=QWEN3_8B)
+    w.v_cache[w.block_table[w.seq_ids[0], 0].long(), 1, 2, 0, 3] = float("inf")
+    o = run_attention(w, 1)[0].view(-1, 8, 4, 128)
+    want = torch.zeros_like(o, dtype=torch.bool)
+    want[:, 2, :, 3] = True
+    assert torch.equal(torch.isposinf(o), want) and not torch.isnan(o).any()
+
+
 def test_attention_every_layer_and_repeatable(gpu):
     """Every layer checks against the oracle; a repeated call gives the same
     bits (every output is summed in a fixed order, whatever the timing)."""
