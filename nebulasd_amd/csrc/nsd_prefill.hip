@@ -478,7 +478,9 @@ int launch_prefill(PrefillArgs args, hipStream_t stream) {
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, C::lds_bytes);
   if (attr != hipSuccess) return fail(NSD_ERR_HIP, "prefill_attention: LDS attribute: %s", hipGetErrorString(attr));
   args.positions = C::rows / args.gqa;
-  args.q_blocks = (args.max_seqlen + args.positions - 1) / args.positions;
+  // no prompt is longer than the call: its end is cut there
+  const int longest = (int)std::min<int64_t>(args.max_seqlen, args.total_tokens);
+  args.q_blocks = (int)(((int64_t)longest + args.positions - 1) / args.positions);
   // Without a prompt order and with a lane for every prompt, the workgroups
   // find the non-empty blocks themselves (at most one part block a prompt);
   // else every (block level, prompt) pair has one, and those past their
@@ -488,7 +490,6 @@ int launch_prefill(PrefillArgs args, hipStream_t stream) {
   int64_t items = (int64_t)args.q_blocks * args.n_seqs;
   if (args.compact) items = std::min<int64_t>(items, args.total_tokens / args.positions + args.n_seqs);
   const int64_t grid = items * args.hkv;
-  if (grid > INT32_MAX) return fail(NSD_ERR_UNSUPPORTED, "prefill_attention: grid of %lld workgroups", (long long)grid);
   hipLaunchKernelGGL(prefill_attn_kernel<C>, dim3((unsigned)grid), dim3(C::threads), C::lds_bytes, stream, args);
   return launch_status("prefill_attention");
 }
@@ -534,6 +535,9 @@ extern "C" int nsd_prefill_attention(const void* q, const void* k, const void* v
   args.gqa = gqa;
   args.max_seqlen = max_seqlen;
   args.scale_log2 = softmax_scale * 1.4426950408889634f;
+  const int64_t positions = PrefillWide::rows / gqa;
+  const int64_t grid = (max_seqlen + positions - 1) / positions * n_seqs * num_kv_heads;
+  if (grid > INT32_MAX) return fail(NSD_ERR_UNSUPPORTED, "prefill_attention: grid of %lld workgroups", (long long)grid);
   // Workgroups of the wide shape that have work (the last block of a prompt
   // half full on average): up to nine for four compute units, the narrow one.
   int cus = 0;

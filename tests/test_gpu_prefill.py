@@ -103,6 +103,23 @@ def test_prefill_prompt_counts(gpu, n, long):
     assert (o[:skip] == 7).all() and (lse[:skip] == 7).all()
 
 
+@pytest.mark.parametrize("n", [3, 70], ids=["kernel order", "prompt order"])
+def test_prefill_length_bound_far_above_the_prompts(gpu, n):
+    """A bound of 2^20 positions (a model's longest) gives the exact bound's
+    bits: no workgroups for positions that the call's tokens cannot reach.  A
+    bound whose grid would not fit is refused."""
+    w = make_prefill_workload("prefill_draft", n, device=gpu, lens=[5 + 7 * (i % 9) for i in range(n)])
+    scale = w.spec.head_dim ** -0.5
+    outs = [flash_attn_varlen_func(w.q, w.k, w.v, w.cu_seqlens, w.cu_seqlens, mx, mx, softmax_scale=scale,
+                                   validate=True) for mx in (max(w.lens), 1 << 20)]
+    assert torch.equal(*outs)
+    if n > 64:
+        from nebulasd_amd import _lib
+
+        with pytest.raises(_lib.NativeLibraryError, match="grid"):
+            flash_attn_varlen_func(w.q, w.k, w.v, w.cu_seqlens, w.cu_seqlens, 2**31 - 1, 2**31 - 1, softmax_scale=scale)
+
+
 def test_prefill_matches_torch_sdpa_loop(gpu):
     """The reference's own formulation on the same GPU (transformer_layer.py:7-32):
     per-prompt scaled_dot_product_attention(is_causal=True) after
