@@ -393,8 +393,9 @@ extern "C" int nsd_rmsnorm_inplace(void* x, const void* w, int64_t n_rows, int64
                        eps);
     return launch_status("rmsnorm");
   }
-  // a workgroup per row from the width on where its 256 threads have a vector each
-  if (vectors && hidden % 8 == 0 && hidden >= 1024 && hidden <= 8 * 256 * kRowVecs) {
+  // a workgroup per row from the width on where its 256 threads have a vector
+  // each, while the launch's threads stay below 2^32
+  if (vectors && hidden % 8 == 0 && hidden >= 1024 && hidden <= 8 * 256 * kRowVecs && n_rows < (1 << 24)) {
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3((unsigned)n_rows), dim3(256), 0, as_stream(stream),
                        static_cast<u32x4*>(x), static_cast<const u32x4*>(w), (int)(hidden / 8), eps);
     return launch_status("rmsnorm");
