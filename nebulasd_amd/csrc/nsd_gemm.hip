@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
 // ---- large column tiles and the gated projection ---------------------------
 //
 // kProducers waves bring the unit's W rows and x through LDS and do nothing
-// else; NW x MW x KG consumer waves compute.  Work goes in k blocks of KS: an
+// else; NW x MW consumer waves compute.  Work goes in k blocks of KS: an
 // x slab (16 MT rows x KS) and SUB = TN / RS steps, each a slot of RS weight
 // rows x KS; a block's slab is issued with its first step.  With KS = 256 an
 // instruction brings 512-byte runs of two rows: the W stream of the Qwen3-8B
@@ -195,10 +195,11 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
 // 34.3 in 1 KB runs, whatever the depth (48 to 144 KB in flight per CU), so
 // the ring is three slots and the LDS goes to x.  The x slabs cost the stream
 // under 2 us: the same x loaded to registers by the consumers, 64-byte runs of
-// 16 rows, cost 12.  Consumer (ng, mg, kg) takes the slot's tiles ng, ng + NW,
-// ..., the row tiles mg, mg + MW, ... and the kg-th of KG parts of the block's
-// k, with its x operands kept in registers over the block's steps where they
-// fit; only KG > 1 (one unit tile and few rows) needs a sum across waves.
+// 16 rows, cost 12.  Consumer (ng, mg) takes the slot's tiles ng, ng + NW, ...
+// and the row tiles mg, mg + MW, ... over all of the block's k, with its x
+// operands kept in registers over the block's steps where they fit.  Every sum
+// runs over k in order in one accumulator, so a row's bits do not depend on
+// the rows beside it.
 //
 // Step s may be issued once the consumers have passed the barrier of step
 // s - R + 1, that is once they are done with step s - R, and with the slab of
@@ -206,22 +207,21 @@ __global__ __launch_bounds__(kGemmThreads) void linear_partials_kernel(const f16
 // 1) SUB.
 constexpr int kProducers = 4;
 
-template <int MT_, int TN_, int RS_, int KS_, int R_, int XD_, int NW_, int MW_, int KG_, bool GATED_>
+template <int MT_, int TN_, int RS_, int KS_, int R_, int XD_, int NW_, int MW_, bool GATED_>
 struct StreamShape {
-  static constexpr int MT = MT_, TN = TN_, RS = RS_, KS = KS_, R = R_, XD = XD_, NW = NW_, MW = MW_, KG = KG_;
+  static constexpr int MT = MT_, TN = TN_, RS = RS_, KS = KS_, R = R_, XD = XD_, NW = NW_, MW = MW_;
   static constexpr bool GATED = GATED_;
-  static constexpr int NC = NW * MW * KG, NJ = TN / 16, SUB = TN / RS, JS = RS / 16;
+  static constexpr int NC = NW * MW, SUB = TN / RS, JS = RS / 16;
   static constexpr int kRowB = KS * 2, kSlot = RS * kRowB, kSlab = 16 * MT * kRowB;
   static constexpr int WI = kSlot / 1024 / kProducers, XI = kSlab / 1024 / kProducers;  // instructions per producer
   static constexpr int RPI = 1024 / kRowB;                                              // rows per instruction
-  static constexpr int KW = KS / 32 / KG, JW = JS / NW, MI = (MT + MW - 1) / MW;
+  static constexpr int KW = KS / 32, JW = JS / NW, MI = (MT + MW - 1) / MW;
   static constexpr bool HOIST = SUB > 1 && KW * MI <= 16;  // a block's x operands in at most 64 registers
   static constexpr int kThreads = (kProducers + NC) * kWave;
   static constexpr int kLds = R * kSlot + XD * kSlab;
   static_assert(WI * kProducers * 1024 == kSlot && XI * kProducers * 1024 == kSlab && JW * NW == JS && SUB * RS == TN);
   static_assert(R >= 2 && R - 1 <= (XD - 1) * SUB && kLds <= kGemmLds);
   static_assert(!GATED || (SUB * JW) % 2 == 0);
-  static_assert(KG == 1 || NC * SUB * JW * MI * 1024 <= kLds);
 };
 
 // Unit u as in linear_partials_kernel, in blocks of KS k.
@@ -298,15 +298,11 @@ __global__ __launch_bounds__(S::kThreads) void stream_gemm_kernel(const f16* __r
         if (issued < steps) issue_step(issued++);
       });
     }
-    if constexpr (S::KG > 1) {  // the consumers' two barriers
-      __syncthreads();
-      __syncthreads();
-    }
     return;
   }
 
   const int c = wave - P;
-  const int ng = c % S::NW, mg = c / S::NW % S::MW, kg = c / (S::NW * S::MW);
+  const int ng = c % S::NW, mg = c / S::NW;
   int xrow[MI];
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
@@ -330,7 +326,7 @@ __global__ __launch_bounds__(S::kThreads) void stream_gemm_kernel(const f16* __r
       slot_no = slot_no + 1 == R ? 0 : slot_no + 1;
 #pragma unroll
       for (int s = 0; s < KW; ++s) {
-        const int ch = (((kg * KW + s) * 4 + lg) ^ lr) << 4;
+        const int ch = ((s * 4 + lg) ^ lr) << 4;
         f16x8 a[JW], b[MI];
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -371,33 +367,10 @@ __global__ __launch_bounds__(S::kThreads) void stream_gemm_kernel(const f16* __r
     }
   };
   constexpr int NT = SUB * JW, OUT = S::GATED ? NT / 2 : NT;  // accumulator tiles, of which stored
-  if constexpr (S::KG == 1) {
 #pragma unroll
-    for (int j = 0; j < OUT; ++j)
+  for (int j = 0; j < OUT; ++j)
 #pragma unroll
-      for (int i = 0; i < MI; ++i) store(j, i, acc[j][i], acc[S::GATED ? j + OUT : j][i]);
-  } else {
-    // the KG waves of a group add their sums in LDS, in kg order
-    constexpr int TW = NT * MI;
-    f32x4* red = reinterpret_cast<f32x4*>(smem_raw) + c % (S::NW * S::MW) * S::KG * TW * kWave;
-    __syncthreads();  // every wave is past its last slot
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int i = 0; i < MI; ++i) red[(kg * TW + j * MI + i) * kWave + lane] = acc[j][i];
-    __syncthreads();
-    auto sum = [&](int t) {
-      f32x4 v = red[t * kWave + lane];
-#pragma unroll
-      for (int q = 1; q < S::KG; ++q) v += red[(q * TW + t) * kWave + lane];
-      return v;
-    };
-#pragma unroll
-    for (int u = 0; u < (OUT * MI + S::KG - 1) / S::KG; ++u) {
-      const int t = u * S::KG + kg;
-      if (t < OUT * MI) store(t / MI, t % MI, sum(t), S::GATED ? sum(t + OUT * MI) : f32x4{});
-    }
-  }
+    for (int i = 0; i < MI; ++i) store(j, i, acc[j][i], acc[S::GATED ? j + OUT : j][i]);
 }
 
 // y[i] = fp16(sum over splits of part[s][i]), eight elements per thread.
@@ -497,9 +470,9 @@ template <int MT, int TN>
 int launch_linear(const GemmArgs& g) {
   constexpr int MW = MT > 1 ? 2 : 1, NW = MT > 1 ? 2 : 4;  // one row tile: the waves split the columns
   if constexpr (TN == 64) {
-    return launch_stream<StreamShape<MT, 64, 64, 128, 3, 3, NW, MW, 1, false>>(g);
+    return launch_stream<StreamShape<MT, 64, 64, 128, 3, 3, NW, MW, false>>(g);
   } else if constexpr (TN == 128) {
-    return launch_stream<StreamShape<MT, 128, 64, 128, 4, 3, NW, MW, 1, false>>(g);
+    return launch_stream<StreamShape<MT, 128, 64, 128, 4, 3, NW, MW, false>>(g);
   } else {
     using S = LinearShape<MT, TN>;
     if (int rc = allow_lds<&linear_partials_kernel<MT, TN>, S::kLds>()) return rc;
@@ -518,17 +491,16 @@ int launch_gated(const GemmArgs& g) {
   constexpr int TN = 32 * PAIRS;
   constexpr int MW = MT > 1 ? 2 : 1;
   if constexpr (PAIRS == 1) {
-    // one slot holds the pair; the waves split the row tiles, or k at one or
-    // two of them
-    constexpr int W = MT >= 3 ? 4 : MT, KG = 4 / W;
+    // one slot holds the pair; a wave takes both of its tiles for every W-th row tile
+    constexpr int W = MT < 4 ? MT : 4;
     if constexpr (MT <= 4)
-      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, 32, 256, 3, 3, 1, W, KG, true>>(g);
-    return launch_stream<StreamShape<MT, TN, 32, 128, 4, 4, 1, W, KG, true>>(g);
+      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, 32, 256, 3, 3, 1, W, true>>(g);
+    return launch_stream<StreamShape<MT, TN, 32, 128, 4, 4, 1, W, true>>(g);
   } else {
     constexpr int RS = PAIRS == 3 ? 48 : 32, NW = RS / 16;
     if constexpr (MT <= 5)
-      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, RS, 256, 3, 2, NW, MW, 1, true>>(g);
-    return launch_stream<StreamShape<MT, TN, RS, 128, 4, 3, NW, MW, 1, true>>(g);
+      if (g.k % 256 == 0) return launch_stream<StreamShape<MT, TN, RS, 256, 3, 2, NW, MW, true>>(g);
+    return launch_stream<StreamShape<MT, TN, RS, 128, 4, 3, NW, MW, true>>(g);
   }
 }
 

@@ -111,6 +111,17 @@ def test_gated_row_tiles(gpu, rows, inter, hidden):
     assert ((out.double() - want).abs() <= 2e-3 * want.abs() + 1e-3).all()
 
 
+@pytest.mark.parametrize("inter,hidden", [(3072, 1024), (3200, 384), (6144, 512), (12288, 768), (12800, 384),
+                                          (1024, 512)], ids=["1pair", "1pair-k128", "2pairs", "3pairs", "4pairs", "ring"])
+def test_gated_row_bits_do_not_depend_on_the_row_count(gpu, inter, hidden):
+    """k is summed in order at every row count: a row has the same bits alone and beside any others."""
+    x = _randn(gpu, 128, hidden, seed=35)
+    w = _randn(gpu, 2 * inter, hidden, seed=36, scale=hidden ** -0.5)
+    want = up_gate_silu_and_mul(x, w)
+    for rows in ROW_EDGES:
+        assert torch.equal(up_gate_silu_and_mul(x[:rows].contiguous(), w), want[:rows]), rows
+
+
 def test_linear_rejects_bad_shapes(gpu):
     x = torch.zeros(2, 256, dtype=torch.float16, device=gpu)
     with pytest.raises(_lib.NativeLibraryError, match="n_out=40"):
