@@ -180,7 +180,8 @@ __device__ inline void merge_row(const AttnArgs& a, int head, int first, int n_s
     for (int u = 0; u < 8; ++u) {
       const int sidx = s0 + u < n_slots ? s0 + u : s0;
       ls[u] = s0 + u < n_slots ? pl[(int64_t)sidx * a.rows_max] : -INFINITY;
-      const f16x8 h = *reinterpret_cast<const f16x8*>(po + sidx * sstride);
+      f16x8 h = *reinterpret_cast<const f16x8*>(po + sidx * sstride);
+      if (s0 + u >= n_slots) h = f16x8{};  // a repeated slot may hold an infinity: 0 * inf
       v0[u] = f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
       v1[u] = f32x4{(float)h[4], (float)h[5], (float)h[6], (float)h[7]};
     }

@@ -128,14 +128,18 @@ def test_attention_merge_of_many_pieces(gpu, model, q_len, ctxs):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
 
 
-@pytest.mark.parametrize("ctx", [1160, 4300, 9000], ids=["9 slots", "34", "64"])
-def test_attention_merge_keeps_an_infinity(gpu, ctx):
+@pytest.mark.parametrize("ctx,slots", [(255, 2), (390, 3), (520, 4), (640, 5), (780, 6), (900, 7), (1023, 8), (1160, 9),
+                                       (4300, 33), (9000, 64)])
+def test_attention_merge_keeps_an_infinity(gpu, ctx, slots):
     """An infinite value of the first token makes that dim of every row of its heads infinite, and nothing
-    else: no thread of the merge multiplies it by the zero weight of a slot that is not there."""
+    else, whatever the slots a thread of the merge takes: none multiplies it by the zero weight of a slot that
+    is not there."""
     w = make_workload("target_verify", 9, device=gpu, pool_blocks=1200, num_layers=2, ctxs=[ctx], q_len=1,
                       model=QWEN3_8B)
     w.v_cache[w.block_table[w.seq_ids[0], 0].long(), 1, 2, 0, 3] = float("inf")
-    o = run_attention(w, 1)[0].view(-1, 8, 4, 128)
+    o, _, st = run_attention(w, 1)
+    assert (planmod.decode_plan(st.attn_plan.host)["combines"][:, 2] == slots).all()
+    o = o.view(-1, 8, 4, 128)
     want = torch.zeros_like(o, dtype=torch.bool)
     want[:, 2, :, 3] = True
     assert torch.equal(torch.isposinf(o), want) and not torch.isnan(o).any()
