@@ -4,6 +4,8 @@
 // All of these move at most a few MB per layer call, so they are
 // launch-latency bound; the design goal is one launch, coalesced 16-byte
 // copies for the cache writes, and wave64 shuffles for the norm reduction.
+#include <algorithm>
+
 #include "nsd_device.h"
 
 // fp32 results are rounded to fp32 and then to fp16, as the reference's
@@ -208,34 +210,24 @@ __global__ __launch_bounds__(256) void rope_kernel(f16* __restrict__ q, f16* __r
   }
 }
 
-// The same for heads of 128, bit for bit: bound by memory, so eight lanes
-// hold a head's two halves in 16-byte vectors (8 heads a wave) and a thread
-// keeps kRopeHeads heads' loads in flight.  Before, 2-byte lanes: 9374 tokens
-// x 24 heads 38.8 us, now 23.2 (4.9 TB/s).
-constexpr int kRopeHeads = 4;
+// The same for heads of 128, bit for bit: bound by memory, and by one trip to
+// it at decode sizes, so eight lanes hold a head's two halves in 16-byte
+// vectors (8 heads a wave), one head a thread.  Four heads a thread took 3.2
+// us at 16 to 80 tokens and gained only at about 150k heads (2000 tokens x 72:
+// 10.7 against 11.7).  x 24 heads, 2-byte lanes and a wave a head -> now: 80
+// tokens 2.3 us both, 320 3.0 -> 2.5, 2000 8.8 -> 4.7, 9000 31.8 -> 18.1.
+constexpr int kRopeHeads = 32;         // a workgroup's heads
+constexpr int64_t kMaxGrid = 1 << 20;  // larger calls loop: a launch's threads stay below 2^32
 __global__ __launch_bounds__(256) void rope_heads_kernel(u32x4* __restrict__ q, u32x4* __restrict__ k,
                                                          const u32x4* __restrict__ cos_t,
                                                          const u32x4* __restrict__ sin_t, uint32_t n_heads,
                                                          uint32_t hq, uint32_t hkv) {
   constexpr int H = kUnits / 2;  // vectors of half a head
   const uint32_t c = threadIdx.x & (H - 1);
-  const uint32_t i0 = blockIdx.x * (32u * kRopeHeads) + (threadIdx.x >> 3);
-  u32x4* at[kRopeHeads];
-  u32x4 lo[kRopeHeads], hi[kRopeHeads], cv[kRopeHeads], sv[kRopeHeads];
-#pragma unroll
-  for (int u = 0; u < kRopeHeads; ++u) {
-    const uint32_t i = min(i0 + 32 * u, n_heads - 1);  // past the end: the last head, not stored
+  for (uint32_t i = blockIdx.x * kRopeHeads + threadIdx.x / H; i < n_heads; i += gridDim.x * kRopeHeads) {
     const uint32_t t = i / (hq + hkv), hd = i - t * (hq + hkv);
-    at[u] = (hd < hq ? q + ((int64_t)t * hq + hd) * kUnits : k + ((int64_t)t * hkv + (hd - hq)) * kUnits) + c;
-    lo[u] = at[u][0];
-    hi[u] = at[u][H];
-    cv[u] = cos_t[(int64_t)t * H + c];
-    sv[u] = sin_t[(int64_t)t * H + c];
-  }
-#pragma unroll
-  for (int u = 0; u < kRopeHeads; ++u) {
-    if (i0 + 32 * u >= n_heads) break;
-    const f16x8 a = h8(lo[u]), b = h8(hi[u]), cs = h8(cv[u]), sn = h8(sv[u]);
+    u32x4* at = (hd < hq ? q + ((int64_t)t * hq + hd) * kUnits : k + ((int64_t)t * hkv + (hd - hq)) * kUnits) + c;
+    const f16x8 a = h8(at[0]), b = h8(at[H]), cs = h8(cos_t[(int64_t)t * H + c]), sn = h8(sin_t[(int64_t)t * H + c]);
     f16x8 o0, o1;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -243,8 +235,8 @@ __global__ __launch_bounds__(256) void rope_heads_kernel(u32x4* __restrict__ q, 
       o0[e] = (f16)(x0 * cc - x1 * ss);
       o1[e] = (f16)(x0 * ss + x1 * cc);
     }
-    at[u][0] = u4(o0);
-    at[u][H] = u4(o1);
+    at[0] = u4(o0);
+    at[H] = u4(o1);
   }
 }
 
@@ -417,10 +409,11 @@ extern "C" int nsd_rotary_embedding_inplace(void* q, void* k, const void* cos_ta
   const int64_t waves = n_tokens * (num_q_heads + num_kv_heads);
   if (head_dim == D && waves <= INT32_MAX && aligned16(q) && aligned16(k) && aligned16(cos_table) &&
       aligned16(sin_table)) {
-    hipLaunchKernelGGL(rope_heads_kernel, dim3((unsigned)((waves + 32 * kRopeHeads - 1) / (32 * kRopeHeads))),
-                       dim3(256), 0, as_stream(stream), static_cast<u32x4*>(q), static_cast<u32x4*>(k),
-                       static_cast<const u32x4*>(cos_table), static_cast<const u32x4*>(sin_table), (uint32_t)waves,
-                       (uint32_t)num_q_heads, (uint32_t)num_kv_heads);
+    const int64_t grid = std::min<int64_t>((waves + kRopeHeads - 1) / kRopeHeads, kMaxGrid);
+    hipLaunchKernelGGL(rope_heads_kernel, dim3((unsigned)grid), dim3(256), 0, as_stream(stream),
+                       static_cast<u32x4*>(q), static_cast<u32x4*>(k), static_cast<const u32x4*>(cos_table),
+                       static_cast<const u32x4*>(sin_table), (uint32_t)waves, (uint32_t)num_q_heads,
+                       (uint32_t)num_kv_heads);
     return launch_status("rope");
   }
   hipLaunchKernelGGL(rope_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0,

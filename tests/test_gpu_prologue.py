@@ -150,7 +150,8 @@ def test_rmsnorm_widths_and_alignments(gpu, rows, hidden, offset):
 
 
 @pytest.mark.parametrize("tokens,hq,hkv,d,offset", [
-    (1, 1, 1, 128, 0), (43, 2, 1, 128, 0), (32, 3, 1, 128, 0), (127, 1, 1, 128, 0), (300, 32, 8, 128, 0),
+    (1, 1, 1, 128, 0), (43, 2, 1, 128, 0), (8, 3, 1, 128, 0), (11, 2, 1, 128, 0), (32, 3, 1, 128, 0),
+    (127, 1, 1, 128, 0), (300, 32, 8, 128, 0),
     (43, 2, 1, 128, 1), (9, 4, 2, 64, 0)])
 def test_rope_head_counts_and_alignments(gpu, tokens, hq, hkv, d, offset):
     g = torch.Generator(device=gpu).manual_seed(tokens + hq)
@@ -169,6 +170,45 @@ def test_rope_head_counts_and_alignments(gpu, tokens, hq, hkv, d, offset):
     ulp_close(q.cpu().numpy(), wq, "rope q")
     ulp_close(k.cpu().numpy(), wk, "rope k")
     assert guards_kept(qbuf, q.numel(), offset) and guards_kept(kbuf, k.numel(), offset)
+
+
+def us_per_call(fn, n=100):
+    """Microseconds a call in a graph of n calls: the fastest of several replays."""
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        fn()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for _ in range(n):
+            fn()
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = float("inf")
+    for _ in range(8):
+        a.record()
+        graph.replay()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+@pytest.mark.parametrize("tokens", [4, 16, 80, 300])
+def test_rope_vector_kernel_is_no_slower_than_the_general_one(gpu, tokens):
+    """At decode and verify sizes, 16-byte aligned heads (the vector kernel) against the same call two bytes off
+    (the general kernel): 0.8 to 1.0 of its time, where a thread of four heads took 1.2 to 1.4."""
+    us = []
+    for offset in (0, 1):
+        q, _ = placed(torch.randn((tokens, 16, 128), device=gpu).half(), offset)
+        k, _ = placed(torch.randn((tokens, 8, 128), device=gpu).half(), offset)
+
+        class S:
+            position_cos = torch.rand((tokens, 64), device=gpu).half()
+            position_sin = torch.rand((tokens, 64), device=gpu).half()
+
+        us.append(us_per_call(lambda: rotary_embedding_inplace(q, k, S)))
+    print(f"rope {tokens} tokens: vector {us[0]:.2f} us, general {us[1]:.2f} us", flush=True)
+    assert us[0] <= 1.12 * us[1]
 
 
 def test_rope_table_matches_oracle(gpu):
