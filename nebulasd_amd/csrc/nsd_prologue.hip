@@ -134,28 +134,23 @@ __device__ inline f16x8 scaled(f16x8 v, float rstd, f16x8 w) {
   return o;
 }
 
-// Head rows (the QK-norm): bound by memory, one read and one write.  16 lanes
-// of 16 bytes hold a row, so a wave covers four and no lane idles, and each
-// thread takes kHeadRows rows with their loads in flight together.  Before,
-// a wave read one row in 2-byte lanes: 150k rows 43.8 us, now 14.6 (5.3 TB/s).
-constexpr int kHeadRows = 4;
+// Head rows (the QK-norm): bound by memory, one read and one write, and by one
+// trip to it at decode sizes.  16 lanes of 16 bytes hold a row, so a wave
+// covers four and no lane idles; a row a thread: four rows a thread took 2.7
+// to 2.9 us at 300 to 3000 rows.  A wave a row in 2-byte lanes -> now: 300
+// rows 2.5 -> 2.2 us, 3000 2.7 -> 2.3, 75k 22.1 -> 9.0.
+constexpr int kNormRows = 16;          // a workgroup's rows
+constexpr int64_t kMaxGrid = 1 << 20;  // larger calls loop: a launch's threads stay below 2^32
 __global__ __launch_bounds__(256) void rmsnorm_heads_kernel(u32x4* __restrict__ x, const u32x4* __restrict__ w,
                                                             int64_t n_rows, float eps) {
   const int c = threadIdx.x & 15;
-  const int64_t row0 = (int64_t)blockIdx.x * (16 * kHeadRows) + (threadIdx.x >> 4);
   const f16x8 wv = h8(w[c]);
-  u32x4 v[kHeadRows];
-#pragma unroll
-  for (int u = 0; u < kHeadRows; ++u) {
-    const int64_t row = row0 + 16 * u;
-    v[u] = x[(row < n_rows ? row : n_rows - 1) * kUnits + c];
-  }
-#pragma unroll
-  for (int u = 0; u < kHeadRows; ++u) {
-    const int64_t row = row0 + 16 * u;
-    const f16x8 xv = h8(v[u]);
-    const float rstd = 1.f / sqrtf(row16_sum(sum_squares(xv)) / (float)D + eps);
-    if (row < n_rows) x[row * kUnits + c] = u4(scaled(xv, rstd, wv));
+  // the 16 lanes of a row, a DPP row, leave together
+  for (int64_t row = (int64_t)blockIdx.x * kNormRows + (threadIdx.x >> 4); row < n_rows;
+       row += (int64_t)gridDim.x * kNormRows) {
+    const f16x8 v = h8(x[row * kUnits + c]);
+    const float rstd = 1.f / sqrtf(row16_sum(sum_squares(v)) / (float)D + eps);
+    x[row * kUnits + c] = u4(scaled(v, rstd, wv));
   }
 }
 
@@ -216,8 +211,7 @@ __global__ __launch_bounds__(256) void rope_kernel(f16* __restrict__ q, f16* __r
 // us at 16 to 80 tokens and gained only at about 150k heads (2000 tokens x 72:
 // 10.7 against 11.7).  x 24 heads, 2-byte lanes and a wave a head -> now: 80
 // tokens 2.3 us both, 320 3.0 -> 2.5, 2000 8.8 -> 4.7, 9000 31.8 -> 18.1.
-constexpr int kRopeHeads = 32;         // a workgroup's heads
-constexpr int64_t kMaxGrid = 1 << 20;  // larger calls loop: a launch's threads stay below 2^32
+constexpr int kRopeHeads = 32;  // a workgroup's heads
 __global__ __launch_bounds__(256) void rope_heads_kernel(u32x4* __restrict__ q, u32x4* __restrict__ k,
                                                          const u32x4* __restrict__ cos_t,
                                                          const u32x4* __restrict__ sin_t, uint32_t n_heads,
@@ -380,9 +374,9 @@ extern "C" int nsd_rmsnorm_inplace(void* x, const void* w, int64_t n_rows, int64
   if (x == nullptr || w == nullptr) return fail(NSD_ERR_INVALID, "rmsnorm: null pointer");
   const bool vectors = aligned16(x) && aligned16(w) && n_rows <= INT32_MAX;
   if (vectors && hidden == D) {
-    hipLaunchKernelGGL(rmsnorm_heads_kernel, dim3((unsigned)((n_rows + 16 * kHeadRows - 1) / (16 * kHeadRows))),
-                       dim3(256), 0, as_stream(stream), static_cast<u32x4*>(x), static_cast<const u32x4*>(w), n_rows,
-                       eps);
+    const int64_t grid = std::min<int64_t>((n_rows + kNormRows - 1) / kNormRows, kMaxGrid);
+    hipLaunchKernelGGL(rmsnorm_heads_kernel, dim3((unsigned)grid), dim3(256), 0, as_stream(stream),
+                       static_cast<u32x4*>(x), static_cast<const u32x4*>(w), n_rows, eps);
     return launch_status("rmsnorm");
   }
   // a workgroup per row from the width on where its 256 threads have a vector
