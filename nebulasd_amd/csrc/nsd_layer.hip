@@ -242,15 +242,19 @@ __device__ inline void rg_wait_n() {
 //
 // A step may be issued R - 1 steps ahead: its slot is free once the consumers
 // are past the step R before, and its slab (read into registers at a block's
-// first step) once they are past the first step of the block XD = 2 before,
-// which asks for 2 subs >= R.  Ranges of fewer steps than that (a vocabulary
-// of a few tiles per CU) are issued a step at a time.
-template <int MT_>
+// first step) once they are past the first step of the block XD before, which
+// asks for XD subs >= R.  Ranges of one step (a vocabulary of at most four
+// tiles per CU: 16,384 rows) take a shape with as many slabs as slots: waiting
+// for each of their steps alone, 4096 x 4096 took 33 / 36 / 39 us at 1 / 80 /
+// 128 rows, now 18 / 24 / 30; 16384 x 4096 37 / 41 / 45, now 30 / 34 / 37.
+template <int MT_, bool ONE_STEP_>
 struct LmShape {
-  static constexpr int MT = MT_, KS = 128, R = 4, XD = 2;
+  static constexpr int MT = MT_, KS = 128;
+  static constexpr bool ONE_STEP = ONE_STEP_;            // ranges of one step
+  static constexpr int R = !ONE_STEP || MT <= 5 ? 4 : 3, XD = ONE_STEP ? R : 2;
   static constexpr int RS = 64;                           // weight rows per step: 16 KB slots
   static constexpr int JS = RS / 16;                      // tiles per step
-  static constexpr int kSubs = 20 / JS;                   // most steps of a group
+  static constexpr int kMinSubs = ONE_STEP ? 1 : 2, kSubs = ONE_STEP ? 1 : 20 / JS;  // steps of a group
   static constexpr int NW = MT <= 2 ? 2 : 1, MW = MT;     // consumer waves: over the step's tiles, over row tiles
   static constexpr int JW = JS / NW, KW = KS / 32;
   static constexpr int kRowB = 2 * KS, kSlot = RS * kRowB, kSlab = 16 * MT * kRowB;
@@ -260,7 +264,7 @@ struct LmShape {
   static constexpr int kKeys = 16 * MT * 8;               // a 64-bit key per row, after the slots
   static constexpr int kLds = R * kSlot + XD * kSlab + kKeys;
   static_assert(XI * kRgProducers * 1024 == kSlab && kLds <= 160 * 1024);
-  static_assert((R - 2) * WI + XI <= 63 && 2 * (R - 2) >= R, "waits");
+  static_assert((R - 2) * (WI + XI) <= 63 && XD * kMinSubs >= R, "waits");
 };
 
 // A lane's running argmax over its logits of one x row, visited in rising
@@ -308,7 +312,7 @@ lm_stream_kernel(const f16* __restrict__ x, const f16* __restrict__ w, int n_row
       int g = 0, kb = 0, sub = 0, blk = 0, slot_no = 0;  // of the next step to issue
       auto issue = [&]() __attribute__((always_inline)) {
         if (sub == 0) {
-          const uint32_t slab = (uint32_t)(uintptr_t)(slabs + (blk & 1) * S::kSlab);
+          const uint32_t slab = (uint32_t)(uintptr_t)(slabs + (blk % S::XD) * S::kSlab);
 #pragma unroll
           for (int i = 0; i < S::XI; ++i) rg_dma<false>(slab + (i * P + wv) * 1024, xsrc[i] + (int64_t)kb * KS);
         }
@@ -330,19 +334,19 @@ lm_stream_kernel(const f16* __restrict__ x, const f16* __restrict__ w, int n_row
           }
         }
       };
-      const bool deep = subs >= R - 2;  // else a step at a time
-      const int depth = deep ? R - 1 : 1;
       int issued = 0;
-      while (issued < depth && issued < steps) {
+      while (issued < R - 1 && issued < steps) {
         issue();
         ++issued;
       }
       int at = 0;  // the awaited step's place in its block
       for (int s = 0; s < steps; ++s) {
         // this wave's part of step s has landed: all but its instructions of
-        // the R - 2 steps after it (one slab among them when the block ends)
-        if (deep && issued - s - 1 >= R - 2) {
-          if (at + R - 2 >= subs) rg_wait_n<(R - 2) * S::WI + S::XI>();
+        // the R - 2 steps after it (one slab among them when the block ends;
+        // a slab with each where a block is a step)
+        if (issued - s - 1 >= R - 2) {
+          if constexpr (S::ONE_STEP) rg_wait_n<(R - 2) * (S::WI + S::XI)>();
+          else if (at + R - 2 >= subs) rg_wait_n<(R - 2) * S::WI + S::XI>();
           else rg_wait_n<(R - 2) * S::WI>();
         } else {
           rg_wait_n<0>();
@@ -370,7 +374,7 @@ lm_stream_kernel(const f16* __restrict__ x, const f16* __restrict__ w, int n_row
     int slot_no = 0, blk = 0;
     for (int g = 0; g < groups; ++g) {
       for (int kb = 0; kb < kbs; ++kb, ++blk) {
-        const lds_char* slab = slabs + (blk & 1) * S::kSlab;
+        const lds_char* slab = slabs + (blk % S::XD) * S::kSlab;
         f16x8 b[KW];
 #pragma unroll
         for (int u = 0; u < SUBS; ++u) {
@@ -466,10 +470,19 @@ void launch_lm(const f16* x, const f16* w, int rows, int hidden, int64_t vocab, 
                      vocab, keys, (int)groups, (int)subs, last_pass);
 }
 
+// The longest of the ranges is one step, or several.
+template <int MT>
+void launch_lm_range(const f16* x, const f16* w, int rows, int hidden, int64_t vocab, uint64_t* keys, bool last_pass,
+                     hipStream_t s) {
+  using One = LmShape<MT, true>;
+  if ((vocab + 15) / 16 <= (int64_t)One::JS * rg_grid()) launch_lm<One>(x, w, rows, hidden, vocab, keys, last_pass, s);
+  else launch_lm<LmShape<MT, false>>(x, w, rows, hidden, vocab, keys, last_pass, s);
+}
+
 template <int... N>
 void launch_lm_any(std::integer_sequence<int, N...>, int mt, const f16* x, const f16* w, int rows, int hidden,
                    int64_t vocab, uint64_t* keys, bool last_pass, hipStream_t s) {
-  ((mt == N + 1 ? launch_lm<LmShape<N + 1>>(x, w, rows, hidden, vocab, keys, last_pass, s) : void()), ...);
+  ((mt == N + 1 ? launch_lm_range<N + 1>(x, w, rows, hidden, vocab, keys, last_pass, s) : void()), ...);
 }
 
 // ---- up/gate projection + SiLU·mul ----------------------------------------

@@ -154,7 +154,8 @@ def test_lm_head_argmax_matches_oracle(gpu, rows, hidden, vocab):
 
 
 @pytest.mark.parametrize("rows", [1, 16, 17, 33, 48, 64, 65, 80, 81, 97, 113, 128])
-@pytest.mark.parametrize("hidden,vocab", [(128, 5), (256, 4096), (384, 8200), (512, 4096 * 20 + 16 * 3), (256, 90001)])
+@pytest.mark.parametrize("hidden,vocab", [(128, 5), (256, 4096), (384, 8200), (512, 4096 * 20 + 16 * 3), (256, 90001),
+                                          (1024, 16384), (1024, 16385)])
 def test_lm_head_row_tiles_and_ranges(gpu, rows, hidden, vocab):
     """Every row-tile count with k blocks of 256 and of 128, one to many steps and groups per range, uneven
     ranges, a last tile that the vocabulary ends in: each row's token is a planted row whose logit stands
@@ -169,6 +170,27 @@ def test_lm_head_row_tiles_and_ranges(gpu, rows, hidden, vocab):
     w[at] = signs[:at.numel()].half()
     x = signs[first].half()
     assert torch.equal(lm_head_argmax(x, w), at[first])
+
+
+def test_lm_head_small_ranges_run_ahead(gpu):
+    """4096 vocab rows, one step of the stream a k block, against the four times larger weight of 16,640 rows, two
+    steps: 0.53 of its time, where a range of one step waited for each step alone and took 0.97."""
+    x = _randn(gpu, 16, 4096, seed=15)
+    us = []
+    for vocab in (4096, 16640):
+        ws = [_randn(gpu, vocab, 4096, seed=16 + i, scale=0.02) for i in range(4)]
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        best = float("inf")
+        for _ in range(6):
+            start.record()
+            for i in range(40):
+                lm_head_argmax(x, ws[i % 4])
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 1e3 / 40)
+        us.append(best)
+    print(f"lm_head 4096 rows {us[0]:.1f} us, 16640 rows {us[1]:.1f} us", flush=True)
+    assert us[0] <= 0.75 * us[1]
 
 
 def test_lm_head_argmax_special_values(gpu):
