@@ -234,8 +234,8 @@ __device__ inline void rg_wait_n() {
 // least: two groups of up to 20 tiles at 151936 rows, x a quarter of the
 // weight's bytes through L2.  us per call at 1 / 80 / 128 rows, before (groups
 // of eight tiles, x loaded to registers by every consumer) -> now: 151936 x
-// 4096 237 / 240 / 293 -> 192 / 206 / 234; 151936 x 1024 75 / 70 / 85 -> 52 /
-// 63 / 70; 32000 x 1024 37 / 22 / 25 -> 17 / 20 / 22.  k blocks of 256 (32
+// 4096 229 / 233 / 281 -> 194 / 197 / 216; 151936 x 1024 75 / 68 / 85 -> 53 /
+// 58 / 70; 32000 x 1024 37 / 22 / 26 -> 17 / 20 / 23.  k blocks of 256 (32
 // rows a slot) ran two to five row tiles at 250-364 us, a fifth slot made
 // ranges of two or three steps serial (32000 rows: 59 -> 71) and gained
 // nothing elsewhere.
@@ -255,7 +255,11 @@ struct LmShape {
   static constexpr int RS = 64;                           // weight rows per step: 16 KB slots
   static constexpr int JS = RS / 16;                      // tiles per step
   static constexpr int kMinSubs = ONE_STEP ? 1 : 2, kSubs = ONE_STEP ? 1 : 20 / JS;  // steps of a group
-  static constexpr int NW = MT <= 2 ? 2 : 1, MW = MT;     // consumer waves: over the step's tiles, over row tiles
+  // Consumer waves over the step's tiles and over row tiles.  A wave alone
+  // with a row tile has all of the step's tiles in a chain: two share them to
+  // five row tiles (the most tried).  48 rows x 4096, 16400 / 151936 vocab
+  // rows 42.1 / 195 -> 38.6 / 192 us; 80 rows 42.2 / 200 -> 39.8 / 197.
+  static constexpr int NW = MT <= 5 ? 2 : 1, MW = MT;
   static constexpr int JW = JS / NW, KW = KS / 32;
   static constexpr int kRowB = 2 * KS, kSlot = RS * kRowB, kSlab = 16 * MT * kRowB;
   static constexpr int RPI = 1024 / kRowB;                // rows per instruction
