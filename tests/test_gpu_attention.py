@@ -110,19 +110,19 @@ def test_attention_long_contexts_wide_groups(gpu, q_len):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("model,q_len,ctxs", [
-    (QWEN3_8B, 1, [1023]), (QWEN3_8B, 1, [1160]),          # 8 and 9 pieces a segment: one thread a row, then four
-    (QWEN3_8B, 9, [4100]), (QWEN3_8B, 5, [4300, 20]),      # 32 and 33: four, then sixteen; a whole segment beside
-    (QWEN3_8B, 1, [9000]), (QWEN3_0_6B, 3, [16000]), (dict(QWEN3_8B, num_key_value_heads=2), 3, [12000])],
-    ids=["8", "9", "32-q9", "33-q5", "64-q1", "64-06b-q3", "128-gqa16-q3"])
-def test_attention_merge_of_many_pieces(gpu, model, q_len, ctxs):
+@pytest.mark.parametrize("model,q_len,ctxs,slots", [
+    (QWEN3_8B, 1, [1023], 8), (QWEN3_8B, 1, [1160], 9),         # one thread a row, then four
+    (QWEN3_8B, 9, [4100], 32), (QWEN3_8B, 5, [4300, 20], 33),   # four, then sixteen; a whole segment beside
+    (QWEN3_8B, 1, [9000], 64), (QWEN3_0_6B, 3, [16000], 64),
+    (dict(QWEN3_8B, num_key_value_heads=2), 3, [12000], 93)],
+    ids=["8", "9", "32-q9", "33-q5", "64-q1", "64-06b-q3", "93-gqa16-q3"])
+def test_attention_merge_of_many_pieces(gpu, model, q_len, ctxs, slots):
     """One request's segments are cut into many pieces: the merge's thread counts per row on both sides of
     their rules, rows that do not fill a workgroup among them."""
     w = make_workload("target_verify", 9, device=gpu, pool_blocks=1200, num_layers=2, ctxs=ctxs, q_len=q_len,
                       model=model)
     o, lse, st = run_attention(w, 1)
-    slots = planmod.decode_plan(st.attn_plan.host)["combines"][:, 2]
-    print("slots per split segment", slots.min(), slots.max(), flush=True)
+    assert (planmod.decode_plan(st.attn_plan.host)["combines"][:, 2] == slots).all()
     check_against_oracle(w, 1, o, lse, f"merge q_len={q_len} ctxs={ctxs}")
     o2, lse2, _ = run_attention(w, 1)
     assert torch.equal(o, o2) and torch.equal(lse, lse2)

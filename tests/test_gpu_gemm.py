@@ -80,13 +80,15 @@ ROW_EDGES = [1, 16, 17, 33, 48, 64, 65, 80, 81, 97, 113, 128]  # both sides of e
 
 
 @pytest.mark.parametrize("rows", ROW_EDGES)
-@pytest.mark.parametrize("n,k", [(16384, 128), (16384, 384), (6144, 2688)], ids=["64-1block", "64-3blocks", "128-5splits"])
-def test_linear_row_tiles(gpu, rows, n, k):
+@pytest.mark.parametrize("n,k,want_splits", [(16384, 128, 1), (16384, 384, 1), (6144, 2688, 5)],
+                         ids=["64-1block", "64-3blocks", "128-5splits"])
+def test_linear_row_tiles(gpu, rows, n, k, want_splits):
     """The large column tiles at every row-tile count: one k block, an odd count, and uneven splits.
     fp32 sums of k products of |x w| ~ 0.03 each: within 1e-5 relative plus the same of the rms sum."""
     x = _randn(gpu, rows, k, seed=31)
     w = _randn(gpu, n, k, seed=32, scale=0.03)
     splits = linear_splits(rows, n, k)
+    assert splits == want_splits
     buf = torch.full((splits * rows * n + n,), 7.0, dtype=torch.float32, device=gpu)
     got = linear_partials(x, w, buf[:splits * rows * n].view(splits, rows, n)).double().sum(0)
     assert bool((buf[splits * rows * n:] == 7.0).all()), "the kernel wrote past the partials"

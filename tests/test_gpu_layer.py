@@ -157,9 +157,10 @@ def test_lm_head_argmax_matches_oracle(gpu, rows, hidden, vocab):
 @pytest.mark.parametrize("hidden,vocab", [(128, 5), (256, 4096), (384, 8200), (512, 4096 * 20 + 16 * 3), (256, 90001),
                                           (1024, 16384), (1024, 16385)])
 def test_lm_head_row_tiles_and_ranges(gpu, rows, hidden, vocab):
-    """Every row-tile count with k blocks of 256 and of 128, one to many steps and groups per range, uneven
-    ranges, a last tile that the vocabulary ends in: each row's token is a planted row whose logit stands
-    clear of the rest (|noise logits| stay under 0.5 sqrt(hidden) < hidden / 2), at the range's edges among others."""
+    """Every row-tile count, one k block to eight, one to many steps and groups per range, uneven ranges, a last
+    tile that the vocabulary ends in: each row's token is a planted row whose logit, hidden, stands clear of the
+    rest (standard deviation 0.04 sqrt(hidden), and sqrt(hidden) for the other planted rows), at the range's edges
+    among others."""
     g = torch.Generator(device=gpu).manual_seed(rows + hidden)
     w = (torch.rand((vocab, hidden), device=gpu, generator=g) - 0.5).half() * 0.125
     at = torch.randint(0, vocab, (rows,), device=gpu, generator=g)
@@ -194,7 +195,7 @@ def test_lm_head_small_ranges_run_ahead(gpu):
 
 
 def test_lm_head_argmax_special_values(gpu):
-    """All logits -inf: index 0; all equal: index 0; the first of several NaN; -0 before +0 stays first."""
+    """All logits -inf: index 0; all equal, from weights of either zero: index 0; the first of several NaN."""
     hidden, vocab = 256, 20000
     w = torch.zeros((vocab, hidden), dtype=torch.float16, device=gpu)
     x = torch.ones((3, hidden), dtype=torch.float16, device=gpu)
@@ -207,6 +208,22 @@ def test_lm_head_argmax_special_values(gpu):
     w[77] = 1.0
     w[[4097, 19999, 12345]] = float("nan")
     assert lm_head_argmax(x, w).tolist() == [4097] * 3
+
+
+@pytest.mark.parametrize("negative", [[0], [0, 1, 2, 3], range(0, 5000), range(1, 20000), range(16, 32)],
+                         ids=["first", "first lane's four", "first 5000", "all but the first", "second tile"])
+def test_lm_head_argmax_of_negative_zeros(gpu, negative):
+    """-0 and +0 logits are equal: the first of them is the token, whichever sign it has.  A -0 logit is a
+    negative sum, -2^-28, that rounds to it (a sum of zeros is +0)."""
+    hidden, vocab = 256, 20000
+    w = torch.zeros((vocab, hidden), dtype=torch.float16, device=gpu)
+    w[list(negative), 0] = -(2.0 ** -14)
+    x = torch.full((3, hidden), 2.0 ** -14, dtype=torch.float16, device=gpu)
+    logits = (x.float() @ w.float().t().contiguous()).half()
+    minus = torch.zeros(vocab, dtype=torch.bool, device=gpu)
+    minus[list(negative)] = True
+    assert (logits == 0).all() and torch.equal(torch.signbit(logits), minus.expand(3, vocab))
+    assert lm_head_argmax(x, w).tolist() == [0, 0, 0]
 
 
 def test_lm_head_argmax_wide_many_rows(gpu):

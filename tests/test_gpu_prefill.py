@@ -23,6 +23,13 @@ pytestmark = pytest.mark.gpu
 EDGE_LENS = [1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100, 127, 128, 129, 255, 256, 257]
 
 
+def narrow_shape(gpu, tokens, n_seqs, hq, hkv):
+    """The kernel shape a call takes: 64-row workgroups up to nine 128-row ones with work for four CUs."""
+    gqa = hq // hkv
+    wide = (tokens * gqa // 128 + n_seqs // 2) * hkv
+    return 64 % gqa == 0 and 4 * wide <= 9 * torch.cuda.get_device_properties(gpu).multi_processor_count
+
+
 def run_prefill(w, validate=True):
     lse = torch.empty(w.q.shape[:2], dtype=torch.float32, device=w.q.device)
     o = flash_attn_varlen_func(w.q, w.k, w.v, w.cu_seqlens, w.cu_seqlens, max(w.lens), max(w.lens),
@@ -70,27 +77,32 @@ def test_prefill_wide_shape_edges(gpu, hq, hkv, fill):
     device, or (128 q-heads on one kv head) a head group that only that shape takes."""
     model = dict(QWEN3_8B, num_attention_heads=hq, num_key_value_heads=hkv)
     lens = EDGE_LENS + [511] * fill
+    assert not narrow_shape(gpu, sum(lens), len(lens), hq, hkv)
     w = make_prefill_workload("prefill_target", 8, device=gpu, lens=lens, model=model)
     o, lse = run_prefill(w)
     check(w, o, lse, f"wide {hq}/{hkv}")
 
 
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65])
-@pytest.mark.parametrize("long", [0, 900], ids=["narrow", "wide"])
-def test_prefill_prompt_counts(gpu, n, long):
-    """Prompts up to a lane each (64) and one more; empty prompts among them, a first prompt that does not start
-    at token 0, and a last one that the tokens cut short: rows of no prompt stay as they were."""
+@pytest.mark.parametrize("shape", ["narrow", "wide"])
+def test_prefill_prompt_counts(gpu, n, shape):
+    """Prompts up to a lane each (64) and one more, in both kernel shapes; empty prompts among them, a first
+    prompt that does not start at token 0, and a last one that the tokens cut short: rows of no prompt stay as
+    they were."""
     rng = np.random.default_rng(n)
-    lens = [int(x) for x in rng.integers(0, 70, n)]
-    lens[n // 2] += long if n < 8 else 0
+    lens = [int(x) for x in rng.integers(0, 30, n)]
     lens[n - 1] += 40
-    if long and n >= 8:
-        lens = [x + 120 for x in lens]
+    if shape == "wide":
+        lens = [x + (120 if n >= 8 else 1300) for x in lens]
+        lens[n // 2] += 100
     lens[0] = 0 if n > 1 else lens[0]
+    hq, hkv = (32, 8) if shape == "narrow" else (64, 8)
+    model = dict(QWEN3_8B, num_attention_heads=hq, num_key_value_heads=hkv)
     skip, cut = 5, 9
-    w = make_prefill_workload("prefill_target", n, device=gpu, lens=[skip] + lens)
+    w = make_prefill_workload("prefill_target", n, device=gpu, lens=[skip] + lens, model=model)
     cu = (w.cu_seqlens[1:]).contiguous()
     t = w.tokens - cut
+    assert narrow_shape(gpu, t, n, hq, hkv) == (shape == "narrow")
     o = torch.full((t,) + w.q.shape[1:], 7.0, dtype=torch.float16, device=gpu)
     lse = torch.full(w.q.shape[:2], 7.0, dtype=torch.float32, device=gpu)[:t].contiguous()
     from nebulasd_amd.kernels.prefill_attn import _launch
