@@ -518,9 +518,14 @@ int with_row_tiles(int rows, F&& f) {
 
 // Up/gate tile pairs per gated unit, or 0 for a shape the ring kernel takes:
 // the most units (the fewest pairs) that one round of the compute units
-// holds.  At seven tenths of them busy the stream still fills the memory
-// (Qwen3-0.6B, 192 units of 256: 6.2 us against 9.8); below that the ring
-// kernel's balanced ranges, which use every compute unit, are left to it.
+// holds.  From seven tenths of them busy the gated units are faster at every
+// row count measured (ring / gated, us at 1 / 64 / 128 rows; 180 units: 2880
+// columns x 1024 5.1 / 9.8 / 15.6 and 4.6 / 6.0 / 8.3, x 4096 13.6 / 23.2 /
+// 39.1 and 10.5 / 14.9 / 23.1; 192: 12288 x 2560 22.7 / 27.5 / 37.9 and 21.1 /
+// 23.8 / 29.6).  Below, the ring kernel's balanced ranges use every compute
+// unit, and it depends on the pairs: 152 units of four pairs (9728 columns) x
+// 2560 19.8 / 26.0 / 36.2 and 22.2 / 25.2 / 32.9, but of one (2432) x 2560 9.5
+// / 17.2 / 28.2 and 7.4 / 10.7 / 16.4; those stay with the ring kernel.
 int gated_pairs(int64_t inter, int cus) {
   for (int pairs = 1; pairs <= 4; ++pairs) {
     if (inter % (16 * pairs)) continue;
