@@ -162,46 +162,45 @@ __device__ inline float rows_sum(float x) {
 // same exp2-domain combine as phase 2 of the reference
 // (paged_attn.py:128-149).  The kernel boundary orders it after every partial
 // store of the attention launch.
+//
+// Threads per (row, 8 dims) of the merge: one while a segment's slots are one
+// round of a thread's loads (8), else four (up to 32 slots) or sixteen.  The
+// merge is latency-bound, and a round is one more trip to memory: one request
+// of 32k tokens, 64 slots a segment, took 8.1 us with one thread in eight
+// rounds and takes 3.9 with sixteen threads in one; 9 to 17 slots (ragged
+// verify) 4.6 either way.
+constexpr int kMergeSlots = 8;
+
 // Row n (of the segment's q_len x GQA rows), dims 8 d8 .. 8 d8 + 7, of a
 // split segment of kv head `head` whose partials sit in slots [first, first
-// + n_slots): the slots folded in slot order with a running max (online
-// log-sum-exp), eight slots' loads in flight at a time, and the row stored.
+// + n_slots), at most kMergeSlots: their loads all in flight, the slots
+// folded in slot order (log-sum-exp) and the row stored.
 __device__ inline void merge_row(const AttnArgs& a, int head, int first, int n_slots, int row_start, int n,
                                  int d8) {
   const f16* po = a.part_o + ((int64_t)first * a.rows_max + n) * D + 8 * d8;
   const float* pl = a.part_lse + (int64_t)first * a.rows_max + n;
   const int64_t sstride = (int64_t)a.rows_max * D;  // elements between slots
+  f32x4 v0[kMergeSlots], v1[kMergeSlots];
+  float ls[kMergeSlots];
+#pragma unroll
+  for (int u = 0; u < kMergeSlots; ++u) {
+    const int sidx = u < n_slots ? u : 0;
+    ls[u] = u < n_slots ? pl[(int64_t)sidx * a.rows_max] : -INFINITY;
+    f16x8 h = *reinterpret_cast<const f16x8*>(po + sidx * sstride);
+    if (u >= n_slots) h = f16x8{};  // a repeated slot may hold an infinity: 0 * inf
+    v0[u] = f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
+    v1[u] = f32x4{(float)h[4], (float)h[5], (float)h[6], (float)h[7]};
+  }
   float M = -INFINITY, W = 0.f;
+#pragma unroll
+  for (int u = 0; u < kMergeSlots; ++u) M = fmaxf(M, ls[u]);  // finite: slot 0 holds token 0, which every row attends
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  for (int s0 = 0; s0 < n_slots; s0 += 8) {
-    f32x4 v0[8], v1[8];
-    float ls[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int sidx = s0 + u < n_slots ? s0 + u : s0;
-      ls[u] = s0 + u < n_slots ? pl[(int64_t)sidx * a.rows_max] : -INFINITY;
-      f16x8 h = *reinterpret_cast<const f16x8*>(po + sidx * sstride);
-      if (s0 + u >= n_slots) h = f16x8{};  // a repeated slot may hold an infinity: 0 * inf
-      v0[u] = f32x4{(float)h[0], (float)h[1], (float)h[2], (float)h[3]};
-      v1[u] = f32x4{(float)h[4], (float)h[5], (float)h[6], (float)h[7]};
-    }
-    float mb = M;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) mb = fmaxf(mb, ls[u]);
-    // slot 0 covers token 0, which every row attends: mb is finite from the
-    // first round on, and M = -inf only there (acc and W are 0)
-    const float scale = exp2f(M - mb);
-    acc0 *= scale;
-    acc1 *= scale;
-    W *= scale;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const float wgt = exp2f(ls[u] - mb);
-      acc0 += v0[u] * wgt;
-      acc1 += v1[u] * wgt;
-      W += wgt;
-    }
-    M = mb;
+  for (int u = 0; u < kMergeSlots; ++u) {
+    const float wgt = exp2f(ls[u] - M);
+    acc0 += v0[u] * wgt;
+    acc1 += v1[u] * wgt;
+    W += wgt;
   }
   const float inv = 1.f / W;
   const int qi = n / a.gqa, gh = n - qi * a.gqa;
@@ -212,14 +211,6 @@ __device__ inline void merge_row(const AttnArgs& a, int head, int first, int n_s
   *reinterpret_cast<f16x8*>(a.o + orow * D + 8 * d8) = hv;
   if (d8 == 0 && a.lse != nullptr) a.lse[orow] = (M + __log2f(W)) * kLn2;
 }
-
-// Threads per (row, 8 dims) of the merge: one while a segment's slots are one
-// round of a thread's loads (8), else four (up to 32 slots) or sixteen.  The
-// merge is latency-bound, and a round is one more trip to memory: one request
-// of 32k tokens, 64 slots a segment, took 8.1 us with one thread in eight
-// rounds and takes 3.9 with sixteen threads in one; 9 to 17 slots (ragged
-// verify) 4.6 either way.
-constexpr int kMergeSlots = 8;
 
 // A partly merged row: running max (log2), sum of weights, 8 dims.
 struct MergeState {
