@@ -494,13 +494,13 @@ void launch_lm_any(std::integer_sequence<int, N...>, int mt, const f16* x, const
 // y[r][j] = fp16(up * fp16(silu(gate))) with up = fp16(x[r] . W[j]) and
 // gate = fp16(x[r] . W[I + j]), W the stacked [2I, hidden] up_gate_proj
 // weight: the reference's up/gate GEMM followed by silu_and_mul, with the
-// same two fp16 roundings, without writing the [rows, 2I] product.  Same
-// main loop as the lm_head kernel: one workgroup per CU owns a balanced
-// range of 16-column output tiles, taken TO at a time; a group's ring slot
-// holds the TO up tiles then the TO gate tiles (32*TO weight rows x 256 B of
-// one k step of 128), brought in by four producer waves with
+// same two fp16 roundings, without writing the [rows, 2I] product, for the
+// shapes that no gated unit takes and for passes past 128 rows.  One workgroup
+// per CU owns a balanced range of 16-column output tiles, taken TO at a time;
+// a ring slot holds the TO up tiles then the TO gate tiles (32*TO weight rows
+// x 256 B of one k step of 128), brought in by four producer waves with
 // global_load_lds_dwordx4; one consumer wave per 16-row tile of x holds its
-// x rows in registers, loaded kUgXAhead steps ahead.  An up tile and its gate
+// x rows in registers, loaded ug_xahead steps ahead.  An up tile and its gate
 // tile land in the same lane layout, so the SiLU·mul runs on the
 // accumulators.  Ring depth grows as the slot shrinks, so every shape keeps
 // about 100 KB in flight per CU.
