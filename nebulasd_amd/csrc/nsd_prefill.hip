@@ -78,7 +78,7 @@ struct PrefillCfg {
 //
 // Wide: 32 rows per wave, 128 per workgroup, three workgroups per compute unit
 // (168 VGPRs).  With the device full the matrix cores and the vector units
-// share out the time (47% and 54% of the SIMD cycles, at the clock that power
+// share out the time (50% and 51% of the SIMD cycles, at the clock that power
 // allows: 1.02 PFLOP/s on two 8k prompts, where the library's 8192^3 matrix
 // product reaches 1.15).
 using PrefillWide = PrefillCfg<2, 4, 32, 1, true, 3, 0>;
