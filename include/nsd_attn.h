@@ -304,7 +304,8 @@ int nsd_paged_attention_noalloc(const void* q, void* o, float* lse, const void* 
  * forward's token count and is cut by slicing q[:num_prefill_tokens],
  * model.py:412-415).  max_seqlen bounds every prompt's length: a longer
  * prompt, a negative start or a decreasing pair sets NSD_STATUS_BAD_SEQ and
- * is not (fully) computed.  Hq/Hkv must divide 128.
+ * is not (fully) computed; without seq_order nor may be a prompt that
+ * overlaps another one after a decreasing pair.  Hq/Hkv must divide 128.
  * seq_order (optional, device int32 [n_seqs]): the prompts longest first (a
  * permutation of 0..n_seqs-1; any order is correct, this one balances the
  * shader engines).  An entry outside [0, n_seqs) sets NSD_STATUS_BAD_SEQ.

@@ -491,7 +491,9 @@ int launch_prefill(PrefillArgs args, hipStream_t stream) {
   // find the non-empty blocks themselves (at most one part block a prompt);
   // else every (block level, prompt) pair has one, and those past their
   // prompt's end exit: 1746 of 4096 for 16 prompts of U[128, 1024], which
-  // held the slots of the first levels.
+  // held the slots of the first levels.  Prompts that overlap, which takes a
+  // (flagged) decreasing pair, may have more blocks than that; a workgroup
+  // that looped over further items would spill (228 bytes a lane).
   args.compact = args.seq_order == nullptr && args.n_seqs <= kWave;
   int64_t items = (int64_t)args.q_blocks * args.n_seqs;
   if (args.compact) items = std::min<int64_t>(items, args.total_tokens / args.positions + args.n_seqs);
