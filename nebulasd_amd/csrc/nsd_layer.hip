@@ -41,6 +41,10 @@ __device__ inline u32x4 as_u4(f16x8 v) { return __builtin_bit_cast(u32x4, v); }
 // and little else, so every load of the row goes out before the first use
 // (SPLITS known at compile time): over four splits, 4 x 1024 3.1 -> 2.6 us, 80 x
 // 4096 5.1 -> 4.8.
+// At about 1000 rows, where loads wait for memory anyway, that order is 2-4%
+// slower than one vector after another and w after the sum (1024 x 2048 3.9 ->
+// 4.1, x 8192 8.5 -> 8.9), which costs 0.15 us at decode rows; from 3000 rows
+// on it is 1-2% faster.
 template <int VPT, int SPLITS>
 __global__ void __launch_bounds__(kNormThreads)
 fused_add_rmsnorm_kernel(f16* __restrict__ x, f16* __restrict__ res, const f16* __restrict__ w, int nvec,
