@@ -221,7 +221,7 @@ def test_rmsnorm_head_rows_kernel_beats_the_general_one(gpu, rows):
         x, _ = placed(torch.randn((rows, 128), device=gpu).half(), offset)
         us.append(us_per_call(lambda: rmsnorm_inplace(x, w, 1e-6)))
     print(f"rmsnorm {rows} head rows: vector {us[0]:.2f} us, general {us[1]:.2f} us", flush=True)
-    assert us[0] <= 0.78 * us[1]
+    assert us[0] <= 0.8 * us[1]
 
 
 def test_rope_table_matches_oracle(gpu):
